@@ -8,14 +8,14 @@
 // contiguous values, or "mn-fast" rows of M/N contiguous values) and the
 // MFMA fragments are read out of whichever layout it is.
 //
-// Tiling: a 256-thread block (4 wave64s as 2 x 2) owns a 128 x 128 or
-// 128 x 64 tile of C (the smaller tile when the larger one cannot give every
-// CU two blocks); each wave owns 2 x 2 (or 2 x 1) MFMA 32x32 blocks.  K
-// advances in slabs of 32 held in double-buffered LDS (72 / 54 KiB, so two
-// blocks fit in one CU's 160 KiB).  The next slab's global loads are issued
-// before the current slab's MFMAs and land in the other LDS buffer
-// afterwards; one barrier per slab.  Interior blocks of aligned operands load
-// without bounds checks (a uniform branch); edge blocks zero-fill.
+// Tiling: products that fill the GPU run on the pipelined kernel: a 256-thread
+// block (4 wave64s as 2 x 2) owns a 128 x 128 tile of C and each wave 2 x 2 MFMA
+// 32x32 blocks; K advances in slabs of 32 held in double-buffered LDS (72 KiB,
+// so two blocks fit in one CU's 160 KiB), one barrier per slab.  Products that
+// do not take tiles of 64, 32 or 16 (gemm_tile.hpp), and choose_tile says which
+// and how K splits.  The generic kernel (128 x 128 or 128 x 64 tiles, every load
+// checked) is left for operands of 4 GiB and more and for the few shapes with
+// less than four floats in a row.
 //
 // Within a slab, MFMA step s (0..15) gives lane half h = lane/32 the k index
 // h*16 + s, for both operands, so a lane's A (or B^T) fragment for the whole
@@ -215,6 +215,8 @@ __device__ __forceinline__ void write_tile(const floatx16 (&acc)[MT][NT], float*
 #undef ORCA_STORE_ACC
 }
 
+#include "gemm_tile.hpp"
+
 // TA: A stored [K][lda] (A^T), else [M][lda].  TB: B stored [N][ldb] (B^T), else [K][ldb].
 // Block tile BM x BN, four waves as 2 x 2, wave tile (BM/2) x (BN/2) = MT x NT
 // MFMA 32x32 blocks.
@@ -334,7 +336,13 @@ __global__ void __launch_bounds__(NTHREADS) gemm_mfma_f32_kernel(GemmParams p) {
 // last MFMAs.  sched_group_barrier interleaves one memory instruction after
 // each MFMA.  L[(t+1)%2] was last read before the barrier of slab t-1, so the
 // store in region A of slab t cannot overwrite fragments still to be read.
-template <bool KFAST>
+// UA: operands with no alignment beyond their floats' own (any M, N, K and leading
+// dimensions).  A whole slab is loaded the same way, 16 bytes at 4-byte addresses; a
+// group of columns that runs past a row's end reads into the next row (columns of C
+// that are never stored).  The chunk's last slab, whole or not, takes load_tail, which
+// keeps the last row's last group and a K that is not a multiple of 4 inside the
+// operand (gemm_tile.hpp, shift_down).
+template <bool KFAST, bool UA>
 struct BufOperand {
   const char* base;  // uniform: the operand's first element
   uint32_t voff[4];  // byte offsets of this thread's four float4s in slab 0
@@ -342,7 +350,7 @@ struct BufOperand {
 
   // Rows (M or N) past `lim_mn` are clamped to the last valid row (or float4),
   // so every load stays inside the operand; they only feed rows / columns of
-  // C that are never stored.  lim_mn is a multiple of 4.
+  // C that are never stored.  Without UA lim_mn is a multiple of 4.
   __device__ __forceinline__ void init(const float* b, int64_t ld, int row0_mn, int lim_mn, int kb) {
     base = reinterpret_cast<const char*>(b);
     const int tid = threadIdx.x;
@@ -353,7 +361,7 @@ struct BufOperand {
       if (KFAST)
         off = (int64_t)min(row0_mn + (idx >> 3), lim_mn - 1) * ld + kb + (idx & 7) * 4;
       else
-        off = (int64_t)(kb + (idx >> 5)) * ld + min(row0_mn + (idx & 31) * 4, lim_mn - 4);
+        off = (int64_t)(kb + (idx >> 5)) * ld + min(row0_mn + (idx & 31) * 4, (lim_mn - 1) & ~3);
       voff[j] = (uint32_t)(off * 4);
     }
     slab_bytes = KFAST ? (uint32_t)(BK * 4) : (uint32_t)(BK * ld * 4);
@@ -362,22 +370,53 @@ struct BufOperand {
   __device__ __forceinline__ void load(int t, floatx4 (&r)[4]) const {
     const char* slab = base + (size_t)slab_bytes * (uint32_t)t;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) r[j] = *reinterpret_cast<const floatx4*>(slab + voff[j]);
+    for (int j = 0; j < 4; ++j) {
+      if (UA)
+        r[j] = *reinterpret_cast<const floatx4_u*>(slab + voff[j]);
+      else
+        r[j] = *reinterpret_cast<const floatx4*>(slab + voff[j]);
+    }
   }
-  // The chunk's last, partial slab: k offsets >= klen (a multiple of 4) are
-  // zero-filled without touching memory.
-  __device__ __forceinline__ void load_tail(int t, int klen, floatx4 (&r)[4]) const {
+  // The chunk's last, partial slab (UA: its last slab): k offsets >= klen are
+  // zero-filled without touching memory past the operand.
+  __device__ __forceinline__ void load_tail(int t, int klen, int64_t ld, int row0_mn, int lim_mn, int kb, int K,
+                                            floatx4 (&r)[4]) const {
     const char* slab = base + (size_t)slab_bytes * (uint32_t)t;
     const int tid = threadIdx.x;
+    if (!UA) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int kk = t * BK + (KFAST ? (tid & 7) * 4 : (tid >> 5) + 8 * j);
-      r[j] = kk < klen ? *reinterpret_cast<const floatx4*>(slab + voff[j]) : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int j = 0; j < 4; ++j) {
+        const int kk = t * BK + (KFAST ? (tid & 7) * 4 : (tid >> 5) + 8 * j);
+        r[j] = kk < klen ? *reinterpret_cast<const floatx4*>(slab + voff[j]) : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+    } else if (KFAST) {
+      const int kk = t * BK + (tid & 7) * 4;
+      const int back = max(0, kb + kk - (K - 4));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const floatx4 v = shift_down(*reinterpret_cast<const floatx4_u*>(slab + voff[j] - 4 * (int64_t)back), back);
+        r[j].x = kk < klen ? v.x : 0.0f;
+        r[j].y = kk + 1 < klen ? v.y : 0.0f;
+        r[j].z = kk + 2 < klen ? v.z : 0.0f;
+        r[j].w = kk + 3 < klen ? v.w : 0.0f;
+      }
+    } else {
+      const int c = min(row0_mn + (tid & 31) * 4, (lim_mn - 1) & ~3);
+      const int dlast = max(0, c + 4 - lim_mn);
+      const size_t limit = ((size_t)(K - 1) * (size_t)ld + (size_t)(c - dlast)) * 4;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int kk = t * BK + (tid >> 5) + 8 * j;
+        const size_t off = (size_t)slab_bytes * (uint32_t)t + voff[j];
+        const floatx4 v = shift_down(*reinterpret_cast<const floatx4_u*>(base + (off < limit ? off : limit)),
+                                     kb + kk == K - 1 ? dlast : 0);
+        r[j] = kk < klen ? v : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
     }
   }
 };
 
-template <bool TA, bool TB, bool COLSUM>
+template <bool TA, bool TB, bool COLSUM, bool UA>
 __global__ void __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2))) gemm_mfma_f32_fast_kernel(GemmParams p) {
   constexpr int BM = 128, BN = 128, MT = 2, NT = 2;
   constexpr int A_TILE = tile_floats(BM), B_TILE = tile_floats(BN);
@@ -389,12 +428,12 @@ __global__ void __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2
   const int bz = blockIdx.z, batch = bz / p.splits, split = bz % p.splits;
   const int kb = split * p.k_chunk;
   const int klen = min(p.K, kb + p.k_chunk) - kb;
-  const int nfull = klen / BK;            // whole slabs
+  const int nfull = UA ? (klen - 1) / BK : klen / BK;  // slabs loaded unchecked
   const int n = (klen + BK - 1) / BK;     // slabs, the last one possibly partial
   const bool do_colsum = COLSUM && blockIdx.y == 0;
 
-  BufOperand<!TA> opa;
-  BufOperand<TB> opb;
+  BufOperand<!TA, UA> opa;
+  BufOperand<TB, UA> opb;
   opa.init(p.A + batch * p.sa, p.lda, m0, p.M, kb);
   opb.init(p.B + batch * p.sb, p.ldb, n0, p.N, kb);
 
@@ -422,8 +461,8 @@ __global__ void __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2
     if (t < nfull) {
       load(t);
     } else {
-      opa.load_tail(t, klen, ra);
-      opb.load_tail(t, klen, rb);
+      opa.load_tail(t, klen, p.lda, m0, p.M, kb, p.K, ra);
+      opb.load_tail(t, klen, p.ldb, n0, p.N, kb, p.K, rb);
     }
   };
   auto frags = [&](const float* s, int half, float (&fa)[MT][8], float (&fb)[NT][8]) {
@@ -674,7 +713,7 @@ __attribute__((amdgpu_waves_per_eu(MODE == BAND_EIGHT ? 2 : 1))) gemm_tn_band_ke
   }
 
   BandOperandA opa;
-  BufOperand<false> opb;
+  BufOperand<false, false> opb;
   opa.init(p.A, p.lda, m0, m_ex, p.M);
   opb.init(p.B, p.ldb, n0, p.N, 0);
 
@@ -723,7 +762,7 @@ __attribute__((amdgpu_waves_per_eu(MODE == BAND_EIGHT ? 2 : 1))) gemm_tn_band_ke
       load(t);
     } else {
       opa.load_tail(t, klen, ra, re);
-      opb.load_tail(t, klen, rb);
+      opb.load_tail(t, klen, p.ldb, n0, p.N, 0, p.K, rb);
     }
   };
   auto frags = [&](const float* s, int half, float (&fa)[MT][8], float (&fb)[8], float (&xa)[XS],
@@ -946,134 +985,8 @@ __global__ void colsum_split_reduce_kernel(const float* __restrict__ part, int s
   out[n] = v;
 }
 
-// Skinny products (few rows, short K, A row-major): C[M, N] = A[M, K] op(B),
-// op(B) = B [K][N] (TB = false) or B stored [N][K] (TB = true).  One 32 x 32
-// tile of C per block of SK_WAVES waves, so an M = 256, N = 1024 product is
-// 256 blocks with no K split.  Wave w multiplies the k range [w kq, (w + 1) kq)
-// straight from global memory in MFMA fragment order: for each group of 8 k,
-// lane (i, h) = (l % 32, l / 32) holds A[m0 + i][k8 + 4h .. + 3] (one float4)
-// and the four B values of the same k for column n0 + i, and MFMA step j
-// (0..3) multiplies k = k8 + 4h + j.  Steps 0 and 2 accumulate into one
-// register block and 1 and 3 into another (two independent chains), added at
-// the end; the waves' tiles are summed through LDS in wave order.  SK_DEPTH
-// groups of loads are in flight while one is multiplied.
-// Rows and columns past M / N are clamped to the last valid one (never
-// stored); k past the wave's range reads as zero.
-struct SkinnyParams {
-  const float* A;
-  const float* B;
-  float* C;
-  int64_t lda, ldb, ldc;
-  int M, N, K, kq;
-  int vec;  // A (and B when TB) rows 16-byte aligned with lda, ldb multiples of 4
-  int epi;
-  const float* bias;
-  const float* mask;
-  int64_t ldmask;
-  float* pre;  // EPI_BIAS_RELU_PRE: acc + bias; EPI_RELU_MASK_PRE: acc (with ldc)
-};
-
-template <bool TB>
-__device__ __forceinline__ void skinny_load(const SkinnyParams& p, int row_a, int col_b, int k, int kend, floatx4& a,
-                                            floatx4& b) {
-  if (p.vec && k + 4 <= kend) {
-    a = *reinterpret_cast<const floatx4*>(p.A + (int64_t)row_a * p.lda + k);
-    if (TB) {
-      b = *reinterpret_cast<const floatx4*>(p.B + (int64_t)col_b * p.ldb + k);
-    } else {
-      const float* bp = p.B + (int64_t)k * p.ldb + col_b;
-      b = floatx4{bp[0], bp[p.ldb], bp[2 * p.ldb], bp[3 * p.ldb]};
-    }
-  } else {
-    float av[4], bv[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bool in = k + e < kend;
-      av[e] = in ? p.A[(int64_t)row_a * p.lda + k + e] : 0.0f;
-      bv[e] = in ? (TB ? p.B[(int64_t)col_b * p.ldb + k + e] : p.B[(int64_t)(k + e) * p.ldb + col_b]) : 0.0f;
-    }
-    a = floatx4{av[0], av[1], av[2], av[3]};
-    b = floatx4{bv[0], bv[1], bv[2], bv[3]};
-  }
-}
-
-constexpr int SK_WAVES = 8;   // waves per skinny block, each an eighth of K
-constexpr int SK_DEPTH = 4;   // 8-k groups of loads in flight per wave
-
-template <bool TB>
-__global__ void __launch_bounds__(64 * SK_WAVES) gemm_skinny_kernel(SkinnyParams p) {
-  __shared__ float red[SK_WAVES][32 * 32];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, i = lane & 31, h = lane >> 5;
-  const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
-  const int row_a = min(m0 + i, p.M - 1), col_b = min(n0 + i, p.N - 1);
-  const int kbeg = w * p.kq, kend = min(p.K, kbeg + p.kq);
-  floatx16 acc0, acc1;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    acc0[r] = 0.0f;
-    acc1[r] = 0.0f;
-  }
-  if (kbeg < kend) {
-    floatx4 a[SK_DEPTH], b[SK_DEPTH];
-#pragma unroll
-    for (int d = 0; d < SK_DEPTH; ++d) skinny_load<TB>(p, row_a, col_b, kbeg + 8 * d + 4 * h, kend, a[d], b[d]);
-    for (int base = kbeg; base < kend; base += 8 * SK_DEPTH) {
-#pragma unroll
-      for (int d = 0; d < SK_DEPTH; ++d) {
-        acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d].x, b[d].x, acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d].y, b[d].y, acc1, 0, 0, 0);
-        acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d].z, b[d].z, acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[d].w, b[d].w, acc1, 0, 0, 0);
-        // refill this slot with the group SK_DEPTH ahead (zeros past the wave's range)
-        skinny_load<TB>(p, row_a, col_b, base + 8 * (d + SK_DEPTH) + 4 * h, kend, a[d], b[d]);
-      }
-    }
-  }
-  // register r of lane (i, h) holds C[(r / 4) * 8 + h * 4 + r % 4][i] of this wave's tile
-#pragma unroll
-  for (int r = 0; r < 16; ++r) red[w][((r >> 2) * 8 + h * 4 + (r & 3)) * 32 + i] = acc0[r] + acc1[r];
-  __syncthreads();
-  // thread t < 256: row t / 8, columns 4 (t % 8) .. + 3
-  if (tid >= 256) return;
-  const int row = tid >> 3, c4 = (tid & 7) * 4;
-  const int m = m0 + row;
-  if (m >= p.M) return;
-  float v[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int o = row * 32 + c4 + e;
-    float t = red[0][o];
-#pragma unroll
-    for (int q = 1; q < SK_WAVES; ++q) t = t + red[q][o];
-    v[e] = t;
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int n = n0 + c4 + e;
-    if (n >= p.N) break;
-    float x = v[e];
-    if (p.epi == ORCA_HIP_EPI_BIAS) {
-      x = x + p.bias[n];
-    } else if (p.epi == ORCA_HIP_EPI_BIAS_RELU) {
-      x = x + p.bias[n];
-      x = x > 0.0f ? x : 0.0f;
-    } else if (p.epi == ORCA_HIP_EPI_RELU_MASK) {
-      x = p.mask[(int64_t)m * p.ldmask + n] > 0.0f ? x : 0.0f;
-    } else if (p.epi == ORCA_HIP_EPI_BIAS_RELU_PRE) {
-      x = x + p.bias[n];
-      p.pre[(int64_t)m * p.ldc + n] = x;
-      x = x > 0.0f ? x : 0.0f;
-    } else if (p.epi == ORCA_HIP_EPI_RELU_MASK_PRE) {
-      p.pre[(int64_t)m * p.ldc + n] = x;
-      x = p.mask[(int64_t)m * p.ldmask + n] > 0.0f ? x : 0.0f;
-    }
-    p.C[(int64_t)m * p.ldc + n] = x;
-  }
-}
-
 inline bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
-// Profiler names: "gemm_<op(A)><op(B)>", "_pipe" for the pipelined 128 x 128 kernel.
 // ---------------------------------------------------------------------------
 // Narrow products, which tile badly on the matrix cores: N <= 16 with a
 // row-major B (X W of a classifier head, X^T dY of its weight gradient) and
@@ -1509,25 +1422,91 @@ __global__ void __launch_bounds__(NW_THREADS, 4) narrow_linear_bw_kernel(NarrowL
                       a.K, a.dH_pre);
 }
 
-const char* kernel_name(bool ta, bool tb, bool pipelined) {
-  static const char* names[2][4] = {{"gemm_nn", "gemm_nt", "gemm_tn", "gemm_tt"},
-                                    {"gemm_nn_pipe", "gemm_nt_pipe", "gemm_tn_pipe", "gemm_tt_pipe"}};
-  return names[pipelined ? 1 : 0][(ta ? 2 : 0) + (tb ? 1 : 0)];
-}
-
 }  // namespace
 
 namespace {
 
 // Kernel, tile and K split of one product.
 struct GemmPlan {
-  bool fast;
-  bool skinny;  // 32 x 32 tiles on gemm_skinny_kernel, no K split
+  bool fast;    // the pipelined 128 x 128 kernel
+  bool ua;      // on operands that are not 16-byte aligned (pipelined and small-tile kernels)
+  int tile;     // 0, or the T x T tile of gemm_tile_kernel
   int band;     // 0, or 1 + the gemm_tn_band_kernel mode of a banded X^T dY (no K split)
   int narrow;   // 0, or a narrow product: 1 NN (N <= 16), 2 NT (K <= 16), 3 TN (N <= 16)
   size_t BM, BN, mt, nt;
   int splits, k_chunk;  // for a narrow TN product: K slices and rows per slice
 };
+
+// Profiler names: "gemm_<op(A)><op(B)>", with "_pipe" on 16-byte aligned operands, "_skinny"
+// for few-row products whose 32 x 32 tiles cover half the CUs or more; plain for 64 x 64
+// tiles, unaligned operands and the generic kernel.
+std::string kernel_name(const GemmPlan& g, bool ta, bool tb, size_t M, size_t cus) {
+  std::string name = std::string("gemm_") + (ta ? "t" : "n") + (tb ? "t" : "n");
+  if (g.tile == 32 && !ta && M <= 256 && 2 * g.mt * g.nt >= cus) return name + "_skinny";
+  return (g.fast || g.tile) && !g.ua && g.tile != 64 ? name + "_pipe" : name;
+}
+
+// The tile and K split of a product on the pipelined or small-tile kernels: the candidate
+// with the least estimated time.  A CU that gets r blocks takes
+//   3 us + r (per block + slabs per block * per slab)
+// and a split adds its reduce launch, 2.4 us and the partial sums at 5 TB/s.  X^T dY is priced
+// with its bias gradient (the plan must not depend on whether that is asked for, so that the
+// product's bits do not): a chain of adds of about 10 ns a row beside the small tiles, 0.19 us
+// a slab folded into the 128 tiles, a launch of its own after a split of those.  The
+// constants are fits to HIP-event times of back-to-back launches on 256 CUs, 66 shapes from
+// 8 x 603 x 240 to 2048^3 in all layouts, each tile and split forced in turn.  A slab is 16 KiB
+// of each operand; small tiles pay for row-major ("mn-fast") operands, whose rows of 16 or 32
+// floats take a memory line each, and more when those rows are not 16-byte aligned.  What the
+// small tiles lose per multiply they win by covering the CUs: 64 x 128 x 784 takes 5.3 us on
+// 32 tiles of 16 (13.7 us on one tile of 128 with K split nine ways), 256 x 1024 x 1024 takes
+// 9.3 us on 256 tiles of 32, 1024^3 takes 22 us on 256 tiles of 64 (27.8 us split four ways);
+// from about 230 tiles of 128 on nothing beats those (2048^3: 123 us, tiles of 64: 137).
+// A split's chunks are even runs of slabs; only splits that fill the CUs once or twice
+// are tried.
+void choose_tile(orca_hip_ctx* ctx, GemmPlan& g, bool trans_a, bool trans_b, size_t M, size_t N, size_t K,
+                 size_t batch) {
+  struct Form {
+    int tile;
+    size_t slab_k;
+    double block_us;
+    double slab_us[2][3];  // [unaligned operands][row-major operands: NT; NN, TT; TN]
+  };
+  static constexpr Form forms[4] = {{16, 256, 0.4, {{0.50, 0.60, 0.95}, {0.55, 0.70, 1.05}}},
+                                    {32, 128, 0.5, {{0.64, 0.68, 0.85}, {0.68, 0.90, 0.95}}},
+                                    {64, 64, 1.0, {{1.06, 1.06, 1.06}, {1.06, 1.10, 1.15}}},
+                                    {128, BK, 3.0, {{1.82, 1.82, 1.82}, {1.84, 1.84, 1.84}}}};
+  const size_t target = (size_t)ctx->num_cus;
+  const int mn_fast = (trans_a ? 1 : 0) + (trans_b ? 0 : 1);
+  double best = 1e300;
+  size_t best_chunk = K;
+  for (const Form& f : forms) {
+    if (ctx->gemm_tile_bn && ctx->gemm_tile_bn != f.tile) continue;
+    const size_t t = (size_t)f.tile;
+    const size_t tiles = ((M + t - 1) / t) * ((N + t - 1) / t) * batch, slabs = (K + f.slab_k - 1) / f.slab_k;
+    for (int j = 0; j < 3; ++j) {
+      size_t s = j == 0 ? 1 : std::min<size_t>(std::min<size_t>((size_t)j * target / tiles, slabs / 2), 64);
+      if (ctx->gemm_splits) s = std::min<size_t>((size_t)ctx->gemm_splits, slabs);
+      if (s == 0 || (j > 0 && s == 1)) continue;
+      const size_t per = (slabs + s - 1) / s;
+      s = (slabs + per - 1) / per;
+      const double rounds = (double)((tiles * s + target - 1) / target);
+      double us = 3.0 + rounds * (f.block_us + (double)per * f.slab_us[g.ua ? 1 : 0][mn_fast]);
+      if (s > 1) us += 2.4 + (double)(s + 1) * (double)(batch * M * N) * 4.0 / 5e6;
+      if (mn_fast == 2 && batch == 1) {
+        if (f.tile < 128) us = std::max(us, 4.0 + 0.0105 * (double)K);
+        else us += s > 1 ? 4.0 + 0.009 * (double)K : 0.19 * (double)slabs;
+      }
+      if (us < best) {
+        best = us;
+        g.tile = f.tile == 128 ? 0 : f.tile;
+        g.splits = (int)s;
+        best_chunk = per * f.slab_k;
+      }
+    }
+  }
+  g.fast = !g.tile;
+  g.k_chunk = (int)(g.splits > 1 ? best_chunk : K);
+}
 
 GemmPlan plan_gemm(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t N, size_t K, const float* A,
                    size_t lda, size_t sa, const float* B, size_t ldb, size_t sb, size_t batch,
@@ -1560,26 +1539,29 @@ GemmPlan plan_gemm(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size
   }
   const bool vec_a = aligned16(A) && lda % 4 == 0 && (batch == 1 || sa % 4 == 0);
   const bool vec_b = aligned16(B) && ldb % 4 == 0 && (batch == 1 || sb % 4 == 0);
-  // Products with M, N, K multiples of 4 and 16-byte aligned operands take the
-  // pipelined 128 x 128 kernel, whose per-lane offsets are 32-bit byte offsets
-  // within one operand.
+  // The pipelined and small-tile kernels hold an operand's offsets as 32-bit bytes and
+  // load four floats at a time; the rest (operands of 4 GiB and more, or with fewer
+  // floats than that in a row or column) is the generic kernel's.
   const size_t a_rows = trans_a ? K : M, b_rows = trans_b ? N : K;
-  g.fast = M % 4 == 0 && N % 4 == 0 && K % 4 == 0 && vec_a && vec_b && a_rows * lda * 4 < 0xffffffffull &&
-           b_rows * ldb * 4 < 0xffffffffull && !ctx->gemm_generic_only;
-  // Generic kernel tile: 128 x 128 when that gives every CU a block, else
-  // 128 x 64 (twice the blocks), unless the context fixes it (tuning).
+  auto loads4 = [](bool kfast, size_t lim, size_t k, size_t ld) { return kfast ? k >= 4 : ld >= 4 && (k >= 2 || lim >= 4); };
+  const bool mfma = a_rows * lda * 4 < 0xffffffffull && b_rows * ldb * 4 < 0xffffffffull && loads4(!trans_a, M, K, lda) &&
+                    loads4(trans_b, N, K, ldb) && !ctx->gemm_generic_only;
+  const bool aligned = M % 4 == 0 && N % 4 == 0 && K % 4 == 0 && vec_a && vec_b;
+  g.fast = mfma;
+  g.ua = !aligned;
   const size_t target = (size_t)ctx->num_cus;
   const size_t t128 = ((M + 127) / 128) * ((N + 127) / 128) * batch;
-  int bn = t128 >= target ? 128 : 64;
-  if (ctx->gemm_tile_bn) bn = ctx->gemm_tile_bn;
-  if (g.fast) bn = 128;
+  size_t BM = 128;
+  // Generic kernel tile: 128 x 128 when that gives every CU a block, else
+  // 128 x 64 (twice the blocks).
+  int bn = mfma || t128 >= target ? 128 : 64;
   // A weight gradient X^T dY (no epilogue) whose banded grid is one round between
   // half and all of the CUs (so it takes no K split) runs banded: 112-row tiles for
   // M = 112 R (R <= 7: as many tiles as 128 rows need, each 12.5 % smaller), or
   // eight 96-row bands plus 16 x 16 blocks for M = 768 + E, whichever the context
   // prefers when both apply.
   const size_t band_cols = N / 128;
-  if (g.fast && ctx->gemm_band && trans_a && !trans_b && batch == 1 && epi_kind == ORCA_HIP_EPI_NONE &&
+  if (g.fast && aligned && ctx->gemm_band && trans_a && !trans_b && batch == 1 && epi_kind == ORCA_HIP_EPI_NONE &&
       N % 128 == 0) {
     const size_t r112 = M / BAND_AP;
     const bool rows112 = M % BAND_AP == 0 && r112 >= 1 && r112 <= 7 && r112 * band_cols <= target &&
@@ -1599,52 +1581,26 @@ GemmPlan plan_gemm(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size
       return g;
     }
   }
-  size_t BM = 128;
-  // Short products (K <= 512) whose 128 x 128 grid leaves at least half the
-  // CUs idle take 64 x 64 tiles on the generic kernel instead of splitting K,
-  // when those tiles alone give three quarters of the CUs a block: the K
-  // split's partial sums and their reduce launch are gone (the weight
-  // gradients of a 256-row batch).  With fewer tiles, or a long K, the
-  // generic kernel's K loop costs more than the split saves.
-  const size_t t64 = ((M + 63) / 64) * ((N + 63) / 64) * batch;
-  if (ctx->gemm_small_tiles && K <= 512 && t128 <= target / 2 && 4 * t64 >= 3 * target) {
-    g.fast = false;
-    BM = 64;
-    bn = 64;
-  }
-  // Few rows and a short K (A row-major): when 32 x 32 tiles give between a
-  // half and two blocks per CU, the skinny kernel takes the product whole, with
-  // no K split (with more of its tiles the 128 x 128 split is faster).
-  const size_t t32 = ((M + 31) / 32) * ((N + 31) / 32);
-  if (ctx->gemm_skinny && !trans_a && batch == 1 && BM == 128 && t128 <= target / 2 && M <= 256 && K <= 1024 &&
-      2 * t32 >= target && t32 <= 2 * target) {
-    g.skinny = true;
-    g.fast = false;
-    BM = 32;
-    bn = 32;
+  g.splits = 1;
+  g.k_chunk = (int)K;
+  if (mfma) {
+    choose_tile(ctx, g, trans_a, trans_b, M, N, K, batch);
+    if (g.tile) {
+      BM = (size_t)g.tile;
+      bn = g.tile;
+    }
+  } else if (t128 <= target / 2 && K >= 4 * (size_t)BK) {
+    // the generic kernel splits K when its tiles leave at least half the CUs idle
+    const size_t tiles = ((M + 127) / 128) * ((N + (size_t)bn - 1) / (size_t)bn) * batch;
+    const size_t s = std::max<size_t>(1, std::min<size_t>(std::min<size_t>((target + tiles - 1) / tiles, K / (2 * BK)), 64));
+    const size_t per = ((K + s - 1) / s + BK - 1) / BK * BK;
+    g.splits = (int)((K + per - 1) / per);
+    if (g.splits > 1) g.k_chunk = (int)per;
   }
   g.BM = BM;
   g.BN = (size_t)bn;
   g.mt = (M + BM - 1) / BM;
   g.nt = (N + g.BN - 1) / g.BN;
-  // Split K when the tile grid leaves at least half the CUs idle and K is long
-  // enough (a grid of exactly half the CUs halves its time with two chunks;
-  // between half and all of them a split would not shorten the longest CU).
-  g.splits = 1;
-  const size_t tiles = g.mt * g.nt * batch;
-  if (BM == 128 && !g.skinny && tiles <= target / 2 && K >= 4 * (size_t)BK) {
-    size_t want = (target + tiles - 1) / tiles;
-    size_t max_by_k = K / (2 * BK);
-    g.splits = (int)std::min<size_t>(std::min<size_t>(want, max_by_k), 64);
-    if (g.splits < 1) g.splits = 1;
-  }
-  g.k_chunk = (int)K;
-  if (g.splits > 1) {
-    size_t per = (K + g.splits - 1) / g.splits;
-    per = (per + BK - 1) / BK * BK;
-    g.splits = (int)((K + per - 1) / per);
-    g.k_chunk = (int)per;
-  }
   return g;
 }
 
@@ -1838,43 +1794,6 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
     gemm_narrow(ctx, plan, M, N, K, A, lda, B, ldb, C, ldc, epi);
     return;
   }
-  if (plan.skinny) {
-    SkinnyParams q{};
-    q.A = A;
-    q.B = B;
-    q.C = C;
-    q.lda = (int64_t)lda;
-    q.ldb = (int64_t)ldb;
-    q.ldc = (int64_t)ldc;
-    q.M = (int)M;
-    q.N = (int)N;
-    q.K = (int)K;
-    q.kq = (int)(((K + SK_WAVES - 1) / SK_WAVES + 7) / 8 * 8);
-    q.vec = aligned16(A) && lda % 4 == 0 && (!trans_b || (aligned16(B) && ldb % 4 == 0));
-    q.epi = epi.kind;
-    q.bias = epi.bias;
-    q.mask = epi.mask;
-    q.ldmask = (int64_t)epi.ldmask;
-    q.pre = epi.pre;
-    {
-      std::string pname;
-      if (ctx->prof.enabled)
-        pname = std::string(trans_b ? "gemm_nt_skinny " : "gemm_nn_skinny ") + std::to_string(M) + "x" +
-                std::to_string(N) + "x" + std::to_string(K);
-      ProfScope ps(ctx, pname.c_str(), 2.0 * (double)M * N * K, 4.0 * (double)(M * K + K * N + M * N));
-      dim3 grid((unsigned)plan.nt, (unsigned)plan.mt);
-      if (trans_b)
-        hipLaunchKernelGGL(gemm_skinny_kernel<true>, grid, dim3(64 * SK_WAVES), 0, ctx->stream, q);
-      else
-        hipLaunchKernelGGL(gemm_skinny_kernel<false>, grid, dim3(64 * SK_WAVES), 0, ctx->stream, q);
-      ORCA_HIP_CHECK(hipGetLastError());
-    }
-    if (epi.colsum) {  // only a row-major B has one (the bias gradient of X^T dY, which is not skinny)
-      if (trans_b) fail(ORCA_HIP_ERR_INTERNAL, "gemm colsum epilogue requires row-major B");
-      launch_colsum(ctx, B, K, N, ldb, epi.colsum);
-    }
-    return;
-  }
   const bool fast = plan.fast;
   const int bn = (int)plan.BN;
   const size_t mt = plan.mt, nt = plan.nt;
@@ -1902,7 +1821,10 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
   p.mask = epi.mask;
   p.ldmask = (int64_t)epi.ldmask;
   p.pre = epi.pre;
-  const bool fold_colsum = epi.colsum != nullptr && batch == 1 && !trans_b && (splits == 1 || !epi.exact_colsum);
+  // The small-tile kernel takes exact column sums in blocks of their own, split or not.
+  const bool tile_colsum = plan.tile && epi.colsum != nullptr && batch == 1 && !trans_b;
+  const bool fold_colsum =
+      epi.colsum != nullptr && batch == 1 && !trans_b && !plan.tile && (splits == 1 || !epi.exact_colsum);
   // Split-K partials (and per-split column sums) go to the caller's workspace
   // when it provides one, else to blocks from the context cache.
   const size_t ws_need = plan_workspace_floats(plan, M, N, batch, fold_colsum);
@@ -1917,19 +1839,19 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
       ws = scratch->as<float>();
     }
   }
-  p.colsum = fold_colsum ? (splits > 1 ? ws + batch * (size_t)splits * M * N : epi.colsum) : nullptr;
+  p.colsum = tile_colsum ? epi.colsum : fold_colsum ? (splits > 1 ? ws + batch * (size_t)splits * M * N : epi.colsum) : nullptr;
   p.vec_a = vec_a;
   p.vec_b = vec_b;
   p.C = splits > 1 ? ws : C;
 
-  dim3 grid((unsigned)nt, (unsigned)mt, (unsigned)(batch * splits));
+  dim3 grid((unsigned)nt, (unsigned)(mt + (tile_colsum ? 1 : 0)), (unsigned)(batch * splits));
   {
     // Profiler records carry the product's shape: "gemm_tn_pipe 4096x4096x1024".
     std::string pname;
     if (ctx->prof.enabled) {
       pname = std::string(plan.band == 1 + BAND_EIGHT     ? "gemm_tn_band8"
                           : plan.band == 1 + BAND_ROWS112 ? "gemm_tn_band112"
-                                                          : kernel_name(trans_a, trans_b, fast)) +
+                                                          : kernel_name(plan, trans_a, trans_b, M, ctx->num_cus)) +
               " " +
               std::to_string(M) + "x" + std::to_string(N) + "x" + std::to_string(K);
       if (batch > 1) pname += "x" + std::to_string(batch);
@@ -1945,17 +1867,34 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
     else if (trans_a && !trans_b) GEMM_LAUNCH(BM_, BN_, true, false); \
     else GEMM_LAUNCH(BM_, BN_, true, true);                          \
   } while (0)
-#define FAST_LAUNCH(TA_, TB_, CS_)                                                                        \
-  do {                                                                                                     \
-    if (bind)                                                                                              \
-      hipExtLaunchKernelGGL((gemm_mfma_f32_fast_kernel<TA_, TB_, CS_>), grid, dim3(NTHREADS), 0, ctx->stream, \
-                            nullptr, epi.done, 0, p);                                                      \
-    else                                                                                                   \
-      hipLaunchKernelGGL((gemm_mfma_f32_fast_kernel<TA_, TB_, CS_>), grid, dim3(NTHREADS), 0, ctx->stream, p); \
+    // The pipelined and small-tile kernels are the product's last launch unless a
+    // split reduce or a separate column sum follows.
+    const bool bind = epi.done && splits == 1 && (!epi.colsum || fold_colsum || tile_colsum);
+    auto launch = [&](auto kernel) {
+      if (bind)
+        hipExtLaunchKernelGGL(kernel, grid, dim3(NTHREADS), 0, ctx->stream, nullptr, epi.done, 0, p);
+      else
+        hipLaunchKernelGGL(kernel, grid, dim3(NTHREADS), 0, ctx->stream, p);
+    };
+#define FAST_LAUNCH(TA_, TB_, CS_)                                     \
+  do {                                                                 \
+    if (plan.ua) launch(gemm_mfma_f32_fast_kernel<TA_, TB_, CS_, true>); \
+    else launch(gemm_mfma_f32_fast_kernel<TA_, TB_, CS_, false>);        \
   } while (0)
-    // The pipelined kernel is the product's last launch unless a split
-    // reduce or a separate column sum follows it.
-    const bool bind = epi.done && splits == 1 && (!epi.colsum || fold_colsum);
+#define TILE_LAUNCH(T_)                                                             \
+  do {                                                                              \
+    if (plan.ua) {                                                                  \
+      if (!trans_a && !trans_b) launch(gemm_tile_kernel<T_, false, false, true>);   \
+      else if (!trans_a) launch(gemm_tile_kernel<T_, false, true, true>);           \
+      else if (!trans_b) launch(gemm_tile_kernel<T_, true, false, true>);           \
+      else launch(gemm_tile_kernel<T_, true, true, true>);                          \
+    } else {                                                                        \
+      if (!trans_a && !trans_b) launch(gemm_tile_kernel<T_, false, false, false>);  \
+      else if (!trans_a) launch(gemm_tile_kernel<T_, false, true, false>);          \
+      else if (!trans_b) launch(gemm_tile_kernel<T_, true, false, false>);          \
+      else launch(gemm_tile_kernel<T_, true, true, false>);                         \
+    }                                                                               \
+  } while (0)
 #define BAND_LAUNCH(MODE_, CS_)                                                                          \
   do {                                                                                                    \
     const dim3 threads(CS_ && MODE_ == BAND_EIGHT ? NTHREADS + 64 : NTHREADS);                           \
@@ -1984,8 +1923,11 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
       else if (trans_a && !trans_b && cs) FAST_LAUNCH(true, false, true);
       else if (trans_a && !trans_b) FAST_LAUNCH(true, false, false);
       else FAST_LAUNCH(true, true, false);
-    } else if (plan.BM == 64) {
-      GEMM_DISPATCH(64, 64);
+    } else if (plan.tile) {
+      bound = bind;
+      if (plan.tile == 16) TILE_LAUNCH(16);
+      else if (plan.tile == 32) TILE_LAUNCH(32);
+      else TILE_LAUNCH(64);
     } else if (bn == 128) {
       GEMM_DISPATCH(128, 128);
     } else {
@@ -1993,6 +1935,7 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
     }
 #undef BAND_LAUNCH
 #undef FAST_LAUNCH
+#undef TILE_LAUNCH
 #undef GEMM_DISPATCH
 #undef GEMM_LAUNCH
     ORCA_HIP_CHECK(hipGetLastError());
@@ -2038,7 +1981,7 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
     ORCA_HIP_CHECK(hipGetLastError());
   }
   // Column sums that the GEMM could not fold in (batched, or B^T storage).
-  if (epi.colsum && !fold_colsum) {
+  if (epi.colsum && !fold_colsum && !tile_colsum) {
     if (batch != 1) fail(ORCA_HIP_ERR_INTERNAL, "gemm colsum epilogue requires batch == 1");
     if (trans_b) fail(ORCA_HIP_ERR_INTERNAL, "gemm colsum epilogue requires row-major B");
     launch_colsum(ctx, B, K, N, ldb, epi.colsum);

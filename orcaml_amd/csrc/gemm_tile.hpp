@@ -1,0 +1,379 @@
+// Small-tile fp32 MFMA product kernel (part of gemm.hip, which defines
+// GemmParams and the vector types): T x T tiles of C for T = 16, 32 or 64.
+//
+// What bounds the products it takes is latency and the number of CUs at work,
+// not the matrix cores: a 64 x 128 x 784 product is one 128 x 128 tile, whose
+// 25 slabs keep one CU's MFMA pipes busy for 43 us, but 32 tiles of 16 x 16.
+// A block is four waves and a slab of KS = 4096 / T k-values (16 KiB of each
+// operand, four float4 per thread and operand whatever T is), so the layout of
+// a load is the same work per thread in every form:
+//   T = 16  four waves split the slab's k range (64 each, v_mfma_f32_16x16x4f32)
+//   T = 32  four waves split it too (32 each, v_mfma_f32_32x32x2f32)
+//   T = 64  2 x 2 waves, each a 32 x 32 block over the whole slab
+// A wave sums its even and odd MFMA steps apart (two independent chains).  The
+// split forms add their four waves' blocks in wave order through LDS.
+//
+// Two slabs are in flight in registers while one is multiplied out of double-
+// buffered LDS.  Every load is unconditional: addresses past an operand's end
+// are clamped into it, and what lies past the k range is zeroed when the slab
+// is stored to LDS.  A loop without branches around loads keeps the waits
+// exact (the wait before an LDS store leaves the next slab's loads in flight)
+// and the code short, which matters for launches of a few microseconds.
+//
+// Operands need no alignment beyond their floats' own (UA): the hardware takes
+// 16-byte loads at 4-byte addresses.  In a row-major ("mn-fast") operand a
+// group of four columns may then run past the row's end into the next row,
+// whose values only feed columns of C that are never stored; only in the very
+// last row is it moved back to the operand's end and shifted into place, as is
+// the last group of a k-fast row when K is not a multiple of 4.
+
+typedef floatx4 floatx4_u __attribute__((aligned(4)));
+
+// The four floats that start d places into v (d = 0 .. 3; the rest is don't care).
+__device__ __forceinline__ floatx4 shift_down(const floatx4& v, int d) {
+  floatx4 x;
+  x.x = d == 0 ? v.x : d == 1 ? v.y : d == 2 ? v.z : v.w;
+  x.y = d == 0 ? v.y : d == 1 ? v.z : v.w;
+  x.z = d == 0 ? v.z : v.w;
+  x.w = v.w;
+  return x;
+}
+
+template <int T, bool KFAST, bool UA>
+struct TileOperand {
+  static constexpr int KS = 4096 / T;                 // k-values per slab
+  static constexpr int PITCH = KS + 4;                // floats per k-fast LDS row
+  static constexpr int GAP = T < 32 ? T : 32;         // mn-fast: extra floats per 16 rows, so the k groups of a
+                                                      // fragment read lie in different banks
+  static constexpr int FLOATS = KFAST ? T * PITCH : KS * T + (KS / 16) * GAP;
+  static constexpr int RSTEP = 1024 / T;              // mn-fast: k rows between a thread's float4s
+
+  const char* base;   // uniform
+  uint32_t voff[4];   // byte offsets of this thread's float4s (k-fast: without the k part)
+  uint32_t limit;     // mn-fast: the largest byte offset a load may have
+  uint32_t step;      // mn-fast: bytes per slab
+  int k0;             // this thread's k in slab 0 (mn-fast: of its first float4)
+  int K, kend;        // k-values of the operand; end of this block's range
+  int dlast;          // mn-fast: places the last row's group is moved back
+
+  static __device__ __forceinline__ int mn_off(int k) { return k * T + (k >> 4) * GAP; }
+
+  // Rows and column groups past `lim` (M or N) become the last valid one.
+  __device__ __forceinline__ void init(const float* src, int64_t ld, int row0, int lim, int kb, int kend_, int K_) {
+    const int tid = threadIdx.x;
+    base = reinterpret_cast<const char*>(src);
+    K = K_;
+    kend = kend_;
+    if (KFAST) {
+      k0 = kb + (tid % (KS / 4)) * 4;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        voff[j] = (uint32_t)((int64_t)min(row0 + (tid + 256 * j) / (KS / 4), lim - 1) * ld * 4);
+    } else {
+      const int c = min(row0 + (tid % (T / 4)) * 4, (lim - 1) & ~3);
+      k0 = kb + tid / (T / 4);
+      dlast = UA ? max(0, c + 4 - lim) : 0;
+      limit = (uint32_t)(((int64_t)(K - 1) * ld + c - dlast) * 4);
+      step = (uint32_t)(KS * ld * 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) voff[j] = (uint32_t)(((int64_t)(k0 + RSTEP * j) * ld + c) * 4);
+    }
+  }
+  __device__ __forceinline__ void load(int t, floatx4 (&r)[4]) const {
+    const uint32_t kc = KFAST ? (uint32_t)min(k0 + t * KS, K - 4) * 4u : 0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t off = KFAST ? voff[j] + kc : min(voff[j] + (uint32_t)t * step, limit);
+      if (UA)
+        r[j] = *reinterpret_cast<const floatx4_u*>(base + off);
+      else
+        r[j] = *reinterpret_cast<const floatx4*>(base + off);
+    }
+  }
+  // Slab t from registers to LDS.  LAST: it may be the block's last slab, zeroed from
+  // kend on (and, UA, shifted where its load was moved back into the operand).
+  template <bool LAST>
+  __device__ __forceinline__ void store(int t, const floatx4 (&r)[4], float* __restrict__ s) const {
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      floatx4 v = r[j];
+      if (KFAST) {
+        const int k = k0 + t * KS;
+        if (LAST && UA) {
+          v = shift_down(v, max(0, k - (K - 4)));
+          v.x = k < kend ? v.x : 0.0f;
+          v.y = k + 1 < kend ? v.y : 0.0f;
+          v.z = k + 2 < kend ? v.z : 0.0f;
+          v.w = k + 3 < kend ? v.w : 0.0f;
+        } else if (LAST) {
+          v = k < kend ? v : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        const int idx = tid + 256 * j;
+        *reinterpret_cast<floatx4*>(s + idx / (KS / 4) * PITCH + idx % (KS / 4) * 4) = v;
+      } else {
+        const int k = k0 + t * KS + RSTEP * j;
+        if (LAST && UA) v = shift_down(v, k == K - 1 ? dlast : 0);
+        if (LAST) v = k < kend ? v : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        *reinterpret_cast<floatx4*>(s + mn_off(tid / (T / 4) + RSTEP * j) + tid % (T / 4) * 4) = v;
+      }
+    }
+  }
+  // The HS k-values from kc on (kc % 16 + HS <= 16) of row (or column) `row`.
+  template <int HS>
+  static __device__ __forceinline__ void frag(const float* __restrict__ s, int row, int kc, float (&f)[HS]) {
+    if (KFAST) {
+      const float* p = s + row * PITCH + kc;
+#pragma unroll
+      for (int q = 0; q < HS / 4; ++q) {
+        const floatx4 v = *reinterpret_cast<const floatx4*>(p + 4 * q);
+        f[4 * q] = v.x;
+        f[4 * q + 1] = v.y;
+        f[4 * q + 2] = v.z;
+        f[4 * q + 3] = v.w;
+      }
+    } else {
+      const float* p = s + mn_off(kc) + row;
+#pragma unroll
+      for (int q = 0; q < HS; ++q) f[q] = p[q * T];
+    }
+  }
+};
+
+// One element's epilogue (C at [m][n] gets v).
+__device__ __forceinline__ void tile_store_one(const GemmParams& p, float* C, int64_t ldc, int epi, int m, int n, float v) {
+  switch (epi) {
+    case ORCA_HIP_EPI_BIAS: v = v + p.bias[n]; break;
+    case ORCA_HIP_EPI_BIAS_RELU:
+      v = v + p.bias[n];
+      v = v > 0.0f ? v : 0.0f;
+      break;
+    case ORCA_HIP_EPI_RELU_MASK: v = p.mask[(int64_t)m * p.ldmask + n] > 0.0f ? v : 0.0f; break;
+    case ORCA_HIP_EPI_BIAS_RELU_PRE:
+      v = v + p.bias[n];
+      p.pre[(int64_t)m * ldc + n] = v;
+      v = v > 0.0f ? v : 0.0f;
+      break;
+    case ORCA_HIP_EPI_RELU_MASK_PRE:
+      p.pre[(int64_t)m * ldc + n] = v;
+      v = p.mask[(int64_t)m * p.ldmask + n] > 0.0f ? v : 0.0f;
+      break;
+    default: break;
+  }
+  C[(int64_t)m * ldc + n] = v;
+}
+
+// Slabs 0 .. n - 1 through two register stages and two LDS buffers: while slab t is
+// used, slab t + 1 moves from its stage to the other buffer and slab t + 3's loads go
+// into that stage (slab t + 2's are in flight in the other one).
+//   load(t, stage), store(t, stage, buffer, last) with stage, buffer and last as
+//   integral constants; begin(): slab 0 is in buffer 0; use(t, buffer, mid, more) calls
+//   mid() where it wants the store and the loads issued and, if more, the block's
+//   barrier after which slab t + 1 is in the other buffer.
+// The loop's own slabs are never the last ones: their stores go unchecked, and every
+// load in it is unconditional (a load behind a branch would make the next store wait
+// for every load in flight).
+template <class Load, class Store, class Begin, class Use>
+__device__ __forceinline__ void slab_pipeline(int n, Load load, Store store, Begin begin, Use use) {
+  constexpr std::integral_constant<int, 0> S0;
+  constexpr std::integral_constant<int, 1> S1;
+  constexpr std::false_type MID;
+  constexpr std::true_type LAST;
+  if (n > 2) {
+    load(0, S0);
+    load(1, S1);
+    store(0, S0, S0, MID);
+    load(2, S0);
+  } else {
+    load(0, S0);
+    if (n > 1) load(1, S1);
+    store(0, S0, S0, LAST);
+  }
+  __syncthreads();
+  begin();
+  int t = 0;
+  for (; t + 4 < n; t += 2) {
+    use(t, S0, [&]() {
+      store(t + 1, S1, S1, MID);
+      load(t + 3, S1);
+    }, true, LAST);
+    use(t + 1, S1, [&]() {
+      store(t + 2, S0, S0, MID);
+      load(t + 4, S0);
+    }, true, LAST);
+  }
+  // 1 .. 4 slabs left: t + 1 and t + 2 are in flight, t + 3 is not loaded yet
+  use(t, S0, [&]() {
+    if (t + 1 < n) store(t + 1, S1, S1, LAST);
+    if (t + 3 < n) load(t + 3, S1);
+  }, t + 1 < n, MID);
+  if (t + 1 >= n) return;
+  use(t + 1, S1, [&]() {
+    if (t + 2 < n) store(t + 2, S0, S0, LAST);
+  }, t + 2 < n, MID);
+  if (t + 2 >= n) return;
+  use(t + 2, S0, [&]() {
+    if (t + 3 < n) store(t + 3, S1, S1, LAST);
+  }, t + 3 < n, MID);
+  if (t + 3 >= n) return;
+  use(t + 3, S1, []() {}, false, MID);
+}
+
+// Grid (N tiles, M tiles [+ 1], batch * splits).  The extra row of blocks, when
+// p.colsum is set (row-major B, one batch entry), takes B's column sums over the
+// whole K range: a block's first T threads add their column's values in
+// ascending k from +0 out of the same LDS slabs (the additions of sum_to_shape,
+// so the same bits), beside the product instead of in a launch after it.
+template <int T, bool TA, bool TB, bool UA>
+__global__ void __launch_bounds__(256, 2) gemm_tile_kernel(GemmParams p) {
+  using OpA = TileOperand<T, !TA, UA>;
+  using OpB = TileOperand<T, TB, UA>;
+  constexpr int KS = OpA::KS;
+  constexpr int RED = T == 64 ? 0 : 4 * T * T;
+  constexpr int SLAB = OpA::FLOATS + OpB::FLOATS;
+  static_assert(2 * SLAB >= RED, "the waves' blocks fit the slab buffers");
+  __shared__ __attribute__((aligned(16))) float smem[2 * SLAB];
+
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int n0 = blockIdx.x * T, m0 = blockIdx.y * T;
+  const int bz = blockIdx.z, batch = bz / p.splits, split = bz % p.splits;
+  floatx4 sa[2][4], sb[2][4];  // the register stages
+
+  if (!TB && m0 >= p.M) {  // the column sums
+    if (bz) return;
+    OpB ob;
+    ob.init(p.B, p.ldb, n0, p.N, 0, p.K, p.K);
+    float cs = 0.0f;
+    slab_pipeline(
+        (p.K + KS - 1) / KS, [&](int t, auto st) { ob.load(t, sb[decltype(st)::value]); },
+        [&](int t, auto st, auto buf, auto last) {
+          ob.template store<decltype(last)::value>(t, sb[decltype(st)::value], smem + decltype(buf)::value * SLAB);
+        },
+        []() {},
+        [&](int t, auto buf, auto mid, bool more, auto) {
+          mid();
+          if (tid < T) {
+            const float* s = smem + decltype(buf)::value * SLAB + tid;
+            const int rows = min(KS, p.K - t * KS);
+            // 64 rows' reads ahead of their adds (rows past K are zero): the chain of adds
+            // is what takes the time, about 3 ns a row
+            for (int k = 0; k < rows; k += 64) {
+              float v[64];
+#pragma unroll
+              for (int q = 0; q < 64; ++q) v[q] = s[OpB::mn_off(k + q)];
+#pragma unroll
+              for (int q = 0; q < 64; ++q) cs = cs + v[q];
+            }
+          }
+          if (more) __syncthreads();
+        });
+    if (tid < T && n0 + tid < p.N) p.colsum[n0 + tid] = cs;
+    return;
+  }
+
+  const int kb = split * p.k_chunk, kend = min(p.K, kb + p.k_chunk);
+  const int n = (kend - kb + KS - 1) / KS;
+  OpA oa;
+  OpB ob;
+  oa.init(p.A + batch * p.sa, p.lda, m0, p.M, kb, kend, p.K);
+  ob.init(p.B + batch * p.sb, p.ldb, n0, p.N, kb, kend, p.K);
+
+  constexpr int LW = T == 16 ? 16 : 32;  // lanes of one k group
+  const int i = lane % LW, g = lane / LW;
+  const int ra = T == 64 ? (wave >> 1) * 32 + i : i, rb = T == 64 ? (wave & 1) * 32 + i : i;
+  const int kw = T == 64 ? 16 * g : wave * (KS / 4) + 16 * g;
+
+  using Acc = typename std::conditional<T == 16, floatx4, floatx16>::type;
+  Acc acc[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int r = 0; r < (T == 16 ? 4 : 16); ++r) acc[c][r] = 0.0f;
+
+  constexpr int HS = T == 64 ? 16 : 8;  // MFMA steps in half a slab
+  float fa[2][HS], fb[2][HS];
+  auto frags = [&](const float* s, int half, float (&a)[HS], float (&b)[HS]) {
+    OpA::frag(s, ra, kw + (T == 64 ? 32 : 8) * half, a);
+    OpB::frag(s + OpA::FLOATS, rb, kw + (T == 64 ? 32 : 8) * half, b);
+  };
+  auto mfma = [&](const float (&a)[HS], const float (&b)[HS]) {
+#pragma unroll
+    for (int q = 0; q < HS; ++q) {
+      if constexpr (T == 16)
+        acc[q & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], b[q], acc[q & 1], 0, 0, 0);
+      else
+        acc[q & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], b[q], acc[q & 1], 0, 0, 0);
+    }
+  };
+  // Memory instructions placed among the matrix instructions: per half slab RD fragment
+  // reads, and in the first half eight LDS stores and eight loads.
+  constexpr int RD = (!TA ? HS / 4 : HS / 2) + (TB ? HS / 4 : HS / 2);
+  auto interleave = [&](auto first) {
+#pragma unroll
+    for (int q = 0; q < HS; ++q) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+      if (q < RD) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
+      if (decltype(first)::value && q % (HS / 8) == 0) {
+        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // DS write
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // VMEM read
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  slab_pipeline(
+      n,
+      [&](int t, auto st) {
+        oa.load(t, sa[decltype(st)::value]);
+        ob.load(t, sb[decltype(st)::value]);
+      },
+      [&](int t, auto st, auto buf, auto last) {
+        float* s = smem + decltype(buf)::value * SLAB;
+        oa.template store<decltype(last)::value>(t, sa[decltype(st)::value], s);
+        ob.template store<decltype(last)::value>(t, sb[decltype(st)::value], s + OpA::FLOATS);
+      },
+      [&]() { frags(smem, 0, fa[0], fb[0]); },
+      [&](int, auto buf, auto mid, bool more, auto full) {
+        // the second half's fragments, the store and the loads go under the first half's
+        // multiplications, the barrier and the next slab's first fragments under the second's
+        constexpr int P = decltype(buf)::value;
+        frags(smem + P * SLAB, 1, fa[1], fb[1]);
+        mid();
+        mfma(fa[0], fb[0]);
+        if constexpr (decltype(full)::value) interleave(std::true_type{});
+        if (more) {
+          __syncthreads();
+          frags(smem + (P ^ 1) * SLAB, 0, fa[0], fb[0]);
+        }
+        mfma(fa[1], fb[1]);
+        if constexpr (decltype(full)::value) interleave(std::false_type{});
+      });
+
+  float* C = p.C + batch * p.sc;
+  if (p.splits > 1) C = p.C + (int64_t)bz * p.M * p.N;
+  const int64_t ldc = p.splits > 1 ? p.N : p.ldc;
+  const int epi = p.splits > 1 ? ORCA_HIP_EPI_NONE : p.epi;
+  if constexpr (T == 64) {
+    floatx16 sum[1][1];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sum[0][0][r] = acc[0][r] + acc[1][r];
+    write_tile(sum, C, ldc, epi, m0 + (wave >> 1) * 32, n0 + (wave & 1) * 32, m0 + T <= p.M && n0 + T <= p.N, p);
+  } else {
+    __syncthreads();  // the last slab's fragments are read
+    float* red = smem + wave * T * T;
+#pragma unroll
+    for (int r = 0; r < (T == 16 ? 4 : 16); ++r) {
+      const int row = T == 16 ? g * 4 + r : (r >> 2) * 8 + g * 4 + (r & 3);
+      red[row * T + i] = acc[0][r] + acc[1][r];
+    }
+    __syncthreads();
+    // element e of thread t: row t / T + e * 256 / T, column t % T
+    const int col = n0 + tid % T;
+#pragma unroll
+    for (int e = 0; e < T * T / 256; ++e) {
+      const int o = tid + 256 * e;
+      const int row = m0 + o / T;
+      const float v = ((smem[o] + smem[o + T * T]) + smem[o + 2 * T * T]) + smem[o + 3 * T * T];
+      if (row < p.M && col < p.N) tile_store_one(p, C, ldc, epi, row, col, v);
+    }
+  }
+}

@@ -105,15 +105,14 @@ int orca_hip_ctx_create(int device, orca_hip_ctx** out) {
     ctx->num_cus = prop.multiProcessorCount;
     ctx->alloc.sync_counter = &ctx->host_syncs;
     if (const char* v = std::getenv("ORCA_HIP_GEMM_FAST")) ctx->gemm_generic_only = v[0] == '0';
-    if (const char* v = std::getenv("ORCA_HIP_GEMM_SMALL_TILES")) ctx->gemm_small_tiles = v[0] != '0';
-    if (const char* v = std::getenv("ORCA_HIP_GEMM_SKINNY")) ctx->gemm_skinny = v[0] != '0';
     if (const char* v = std::getenv("ORCA_HIP_GEMM_NARROW")) ctx->gemm_narrow = v[0] != '0';
     if (const char* v = std::getenv("ORCA_HIP_GEMM_BAND")) ctx->gemm_band = v[0] == '0' ? 0 : v[0] == '1' ? 1 : 2;
     if (const char* v = std::getenv("ORCA_HIP_EW_JIT")) ctx->ew_jit_mode = v[0] == '0' ? 0 : v[0] == '2' ? 2 : 1;
     if (const char* v = std::getenv("ORCA_HIP_GEMM_TILE")) {
-      if (std::strcmp(v, "128x128") == 0) ctx->gemm_tile_bn = 128;
-      if (std::strcmp(v, "128x64") == 0) ctx->gemm_tile_bn = 64;
+      const int t = std::atoi(v);
+      if (t == 16 || t == 32 || t == 64 || t == 128) ctx->gemm_tile_bn = t;
     }
+    if (const char* v = std::getenv("ORCA_HIP_GEMM_SPLITS")) ctx->gemm_splits = std::max(0, std::min(64, std::atoi(v)));
     hipError_t e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&ctx->timer_start);
     if (e == hipSuccess) e = hipEventCreate(&ctx->timer_stop);

@@ -205,13 +205,11 @@ struct orca_hip_ctx {
   std::mutex mu;
   // Tuning switches read once when the context is created (environment):
   // ORCA_HIP_GEMM_FAST=0 sends every product through the generic GEMM kernel,
-  // ORCA_HIP_GEMM_TILE=128x128|128x64 fixes the generic kernel's tile (0 = by grid size).
+  // ORCA_HIP_GEMM_TILE=16|32|64|128 fixes the tile of the other products (0 = by the
+  // product's size) and ORCA_HIP_GEMM_SPLITS=n their K split.
   bool gemm_generic_only = false;
   int gemm_tile_bn = 0;
-  // ORCA_HIP_GEMM_SMALL_TILES=0 keeps the K split for small products instead of 64 x 64 tiles.
-  bool gemm_small_tiles = true;
-  // ORCA_HIP_GEMM_SKINNY=0 keeps the K split for few-row products instead of the skinny kernel.
-  bool gemm_skinny = true;
+  int gemm_splits = 0;
   // ORCA_HIP_GEMM_NARROW=0 keeps products with N <= 16 (or K <= 16 against B^T) on the tiled kernels.
   bool gemm_narrow = true;
   // ORCA_HIP_GEMM_BAND: 0 keeps weight gradients X^T dY of 784-like row counts on the

@@ -1,0 +1,146 @@
+"""The small-tile products (T x T tiles, T = 16, 32, 64) and the pipelined 128-tile product on
+operands that are not 16-byte aligned, each tile forced in turn: exact on integers in every
+layout, at the edges of tiles and slabs, with and without a K split, through padded leading
+dimensions and bases off by one float (NaN in the padding and beyond the operand: nothing read
+there may reach C), with the exact column sum and every epilogue."""
+from __future__ import annotations
+
+import ctypes
+import os
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from orcaml_amd import _lib
+from tests.util import int_matrix
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", params=["16/1", "32/1", "64/1", "128/1", "16/2", "32/3", "64/2", "128/3"])
+def tctx(request):
+    """A context whose products take one tile (and K split)."""
+    from orcaml_amd.device import Context
+
+    tile, splits = request.param.split("/")
+    old = {k: os.environ.get(k) for k in ("ORCA_HIP_GEMM_TILE", "ORCA_HIP_GEMM_SPLITS")}
+    os.environ.update(ORCA_HIP_GEMM_TILE=tile, ORCA_HIP_GEMM_SPLITS=splits)
+    try:
+        c = Context(0)
+    finally:
+        for k, v in old.items():
+            if v is None:
+                del os.environ[k]
+            else:
+                os.environ[k] = v
+    yield c
+    c.close()
+
+
+class Operand:
+    """A rows x cols matrix on the device with `pad` extra floats per row and `shift` floats in
+    front, NaN wherever it has no value."""
+
+    def __init__(self, ctx, a, pad, shift):
+        rows, self.ld = a.shape[0], a.shape[1] + pad
+        host = np.full(shift + (rows - 1) * self.ld + a.shape[1] + 64, np.nan, np.float32)
+        view = np.lib.stride_tricks.as_strided(host[shift:], a.shape, (4 * self.ld, 4))
+        view[:] = a
+        self.buf = ctx.upload(host)
+        self.ptr = self.buf.ptr + 4 * shift
+
+
+def product(ctx, ta, tb, A, B, pad=0, shift=0, colsum=False, kind=_lib.EPI_NONE, bias=None, mask=None, pre=False):
+    (M, K), N = A.shape, B.shape[1]
+    a = Operand(ctx, np.ascontiguousarray(A.T) if ta else A, pad, shift)
+    b = Operand(ctx, np.ascontiguousarray(B.T) if tb else B, pad, shift)
+    ldc = N + pad
+    c = ctx.upload(np.full(M * ldc, 7.0, np.float32))
+    keep = [ctx.upload(x) for x in (bias, mask) if x is not None]
+    e = _lib.Epilogue(kind)
+    if bias is not None:
+        e.bias = keep[0].ptr
+    if mask is not None:
+        e.mask, e.ldmask = keep[-1].ptr, N
+    p = ctx.upload(np.full(M * ldc, 7.0, np.float32)) if pre else None
+    if pre:
+        e.pre = p.ptr
+    cs = ctx.alloc(4 * N) if colsum else None
+    if colsum:
+        e.colsum = cs.ptr
+    _lib.call("orca_hip_gemm", ctx.handle, int(ta), int(tb), M, N, K, a.ptr, a.ld, b.ptr, b.ld, c.ptr, ldc,
+              ctypes.byref(e))
+    out = c.download(count=M * ldc).reshape(M, ldc)
+    np.testing.assert_array_equal(out[:, N:], np.full((M, pad), 7.0, np.float32))
+    res = [np.ascontiguousarray(out[:, :N])]
+    if pre:
+        res.append(np.ascontiguousarray(p.download(count=M * ldc).reshape(M, ldc)[:, :N]))
+    if colsum:
+        res.append(cs.download(count=N))
+    return res
+
+
+# M, N, K: one element past, at and short of each tile; K from less than a slab to several, whole
+# and ragged; the fewest floats the kernels take.
+SHAPES = [(17, 17, 17), (16, 32, 64), (15, 33, 255), (31, 65, 257), (64, 128, 784), (63, 129, 513), (129, 127, 300),
+          (132, 260, 36), (1, 18, 4), (4, 20, 1000), (20, 4, 131), (200, 26, 333), (130, 70, 1030)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_every_tile_exact_on_integers(tctx, M, N, K):
+    rng = np.random.default_rng(M * 7 + N * 13 + K)
+    A, B = int_matrix(rng, (M, K)), int_matrix(rng, (K, N))
+    want = (A.astype(np.int64) @ B.astype(np.int64)).astype(np.float32)
+    sums = O.sum_to_shape(B, (1, N)).reshape(N)
+    for pad, shift in ((0, 0), (4, 0), (3, 1), (1, 2)):
+        for ta, tb in ((False, False), (False, True), (True, False), (True, True)):
+            for colsum in (False, True) if not tb else (False,):
+                got = product(tctx, ta, tb, A, B, pad, shift, colsum)
+                np.testing.assert_array_equal(got[0], want, err_msg=f"{ta} {tb} {pad} {shift}")
+                if colsum:
+                    np.testing.assert_array_equal(got[1], sums, err_msg=f"{ta} {tb} {pad} {shift}")
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 65, 257), (128, 64, 512), (130, 70, 300)])
+def test_every_tile_epilogues_and_column_sum_bits(tctx, M, N, K):
+    """Real data: each epilogue is the composed ops on the tile's own product, bit for bit, and the
+    column sum has the bits of sum_to_shape."""
+    rng = np.random.default_rng(M + N + K)
+    A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+    bias, mask = rng.standard_normal(N).astype(np.float32), rng.standard_normal((M, N)).astype(np.float32)
+    mask[::5, ::3] = 0.0
+    prod, cs = product(tctx, False, False, A, B, colsum=True)
+    np.testing.assert_array_equal(cs, O.sum_to_shape(B, (1, N)).reshape(N))
+    # any order of a K-term f32 sum is within K 2^-24 sum |a b|
+    bound = K * 2.0 ** -24 * (np.abs(A.astype(np.float64)) @ np.abs(B.astype(np.float64)))
+    assert (np.abs(prod - A.astype(np.float64) @ B.astype(np.float64)) <= bound).all()
+    biased = O.add(prod, O.expand(bias.reshape(1, N), (M, N)))
+    masked = O.relu_backward(prod, mask)
+    np.testing.assert_array_equal(product(tctx, False, False, A, B, kind=_lib.EPI_BIAS, bias=bias)[0], biased)
+    np.testing.assert_array_equal(product(tctx, False, False, A, B, kind=_lib.EPI_BIAS_RELU, bias=bias)[0],
+                                  O.relu(biased))
+    np.testing.assert_array_equal(product(tctx, False, False, A, B, kind=_lib.EPI_RELU_MASK, mask=mask)[0], masked)
+    for kind, kw, got, kept in ((_lib.EPI_BIAS_RELU_PRE, {"bias": bias}, O.relu(biased), biased),
+                                (_lib.EPI_RELU_MASK_PRE, {"mask": mask}, masked, prod)):
+        c, p = product(tctx, False, False, A, B, kind=kind, pre=True, **kw)
+        np.testing.assert_array_equal(c, got)
+        np.testing.assert_array_equal(p, kept)
+
+
+@pytest.mark.parametrize("batch,M,N,K", [(5, 40, 24, 70), (3, 197, 197, 64), (260, 9, 8, 33)])
+def test_every_tile_batched(tctx, batch, M, N, K):
+    from orcaml_amd.backend import HipBackend
+
+    rng = np.random.default_rng(batch + K)
+    A, B = int_matrix(rng, (batch, M, K)), int_matrix(rng, (batch, K, N))
+    want = (A.astype(np.int64) @ B.astype(np.int64)).astype(np.float32)
+    be = HipBackend(tctx)
+    At, Bt = (np.ascontiguousarray(x.transpose(0, 2, 1)) for x in (A, B))
+    for x, y in ((A, B), (None, B), (A, None), (None, None)):
+        a = be.from_f32_slice((batch, M, K), A) if x is not None else be.transpose(
+            be.from_f32_slice((batch, K, M), At), (batch, K, M), 1, 2)
+        b = be.from_f32_slice((batch, K, N), B) if y is not None else be.transpose(
+            be.from_f32_slice((batch, N, K), Bt), (batch, N, K), 1, 2)
+        got = be.to_f32_vec(be.matmul(a, b, (batch, M, K), (batch, K, N))).reshape(batch, M, N)
+        np.testing.assert_array_equal(got, want)
