@@ -30,6 +30,7 @@
 #include <hip/hip_ext.h>
 
 #include "runtime.hpp"
+#include "slab.hpp"
 
 namespace orca_hip {
 namespace {
@@ -39,9 +40,6 @@ constexpr int LDK = BK + 4;  // pitch of k-fast tile rows (floats)
 constexpr int MN_GAP = 32;   // shift of k-rows 16..31 in mn-fast tiles
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-// Native 4-float vector: copies stay SSA values (HIP's float4 struct copies
-// lower to memcpy, which can pin a register stage in scratch).
-typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 struct GemmParams {
   const float* A;
@@ -341,7 +339,7 @@ __global__ void __launch_bounds__(NTHREADS) gemm_mfma_f32_kernel(GemmParams p) {
 // group of columns that runs past a row's end reads into the next row (columns of C
 // that are never stored).  The chunk's last slab, whole or not, takes load_tail, which
 // keeps the last row's last group and a K that is not a multiple of 4 inside the
-// operand (gemm_tile.hpp, shift_down).
+// operand (slab.hpp, shift_down).
 template <bool KFAST, bool UA>
 struct BufOperand {
   const char* base;  // uniform: the operand's first element
