@@ -1488,7 +1488,8 @@ void choose_tile(orca_hip_ctx* ctx, GemmPlan& g, bool trans_a, bool trans_b, siz
       const size_t per = (slabs + s - 1) / s;
       s = (slabs + per - 1) / per;
       const double rounds = (double)((tiles * s + target - 1) / target);
-      double us = 3.0 + rounds * (f.block_us + (double)per * f.slab_us[g.ua ? 1 : 0][mn_fast]);
+      // one-slab products run four blocks a CU, which hide more of each other's loads and stores
+      double us = 3.0 + rounds * (f.block_us - (slabs == 1 && f.tile < 128 ? 0.15 : 0.0) + (double)per * f.slab_us[g.ua ? 1 : 0][mn_fast]);
       if (s > 1) us += 2.4 + (double)(s + 1) * (double)(batch * M * N) * 4.0 / 5e6;
       if (mn_fast == 2 && batch == 1) {
         if (f.tile < 128) us = std::max(us, 4.0 + 0.0105 * (double)K);
@@ -1879,19 +1880,20 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
     if (plan.ua) launch(gemm_mfma_f32_fast_kernel<TA_, TB_, CS_, true>); \
     else launch(gemm_mfma_f32_fast_kernel<TA_, TB_, CS_, false>);        \
   } while (0)
-#define TILE_LAUNCH(T_)                                                             \
-  do {                                                                              \
-    if (plan.ua) {                                                                  \
-      if (!trans_a && !trans_b) launch(gemm_tile_kernel<T_, false, false, true>);   \
-      else if (!trans_a) launch(gemm_tile_kernel<T_, false, true, true>);           \
-      else if (!trans_b) launch(gemm_tile_kernel<T_, true, false, true>);           \
-      else launch(gemm_tile_kernel<T_, true, true, true>);                          \
-    } else {                                                                        \
-      if (!trans_a && !trans_b) launch(gemm_tile_kernel<T_, false, false, false>);  \
-      else if (!trans_a) launch(gemm_tile_kernel<T_, false, true, false>);          \
-      else if (!trans_b) launch(gemm_tile_kernel<T_, true, false, false>);          \
-      else launch(gemm_tile_kernel<T_, true, true, false>);                         \
-    }                                                                               \
+#define TILE_LAUNCH_UA(T_, UA_, ONE_)                                                     \
+  do {                                                                                    \
+    if (!trans_a && !trans_b) launch(gemm_tile_kernel<T_, false, false, UA_, ONE_>);      \
+    else if (!trans_a) launch(gemm_tile_kernel<T_, false, true, UA_, ONE_>);              \
+    else if (!trans_b) launch(gemm_tile_kernel<T_, true, false, UA_, ONE_>);              \
+    else launch(gemm_tile_kernel<T_, true, true, UA_, ONE_>);                             \
+  } while (0)
+#define TILE_LAUNCH(T_)                                   \
+  do {                                                    \
+    const bool one = K <= 4096 / T_;                      \
+    if (plan.ua && one) TILE_LAUNCH_UA(T_, true, true);   \
+    else if (plan.ua) TILE_LAUNCH_UA(T_, true, false);    \
+    else if (one) TILE_LAUNCH_UA(T_, false, true);        \
+    else TILE_LAUNCH_UA(T_, false, false);                \
   } while (0)
 #define BAND_LAUNCH(MODE_, CS_)                                                                          \
   do {                                                                                                    \
@@ -1934,6 +1936,7 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
 #undef BAND_LAUNCH
 #undef FAST_LAUNCH
 #undef TILE_LAUNCH
+#undef TILE_LAUNCH_UA
 #undef GEMM_DISPATCH
 #undef GEMM_LAUNCH
     ORCA_HIP_CHECK(hipGetLastError());

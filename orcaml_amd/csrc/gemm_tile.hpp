@@ -43,15 +43,18 @@ __device__ __forceinline__ void tile_store_one(const GemmParams& p, float* C, in
 // whole K range: a block's first T threads add their column's values in
 // ascending k from +0 out of the same LDS slabs (the additions of sum_to_shape,
 // so the same bits), beside the product instead of in a launch after it.
-template <int T, bool TA, bool TB, bool UA>
-__global__ void __launch_bounds__(256, 2) gemm_tile_kernel(GemmParams p) {
+// ONE: K is at most one slab.  Without the loop and its second buffer four blocks fit a CU
+// instead of two, so that some load or store while others multiply, and the code is a
+// third as long.
+template <int T, bool TA, bool TB, bool UA, bool ONE>
+__global__ void __launch_bounds__(256, ONE ? 4 : 2) gemm_tile_kernel(GemmParams p) {
   using OpA = TileOperand<T, !TA, UA>;
   using OpB = TileOperand<T, TB, UA>;
   constexpr int KS = OpA::KS;
   constexpr int RED = T == 64 ? 0 : 4 * T * T;
   constexpr int SLAB = OpA::FLOATS + OpB::FLOATS;
-  static_assert(2 * SLAB >= RED, "the waves' blocks fit the slab buffers");
-  __shared__ __attribute__((aligned(16))) float smem[2 * SLAB];
+  static_assert(SLAB >= RED, "the waves' blocks fit a slab buffer");
+  __shared__ __attribute__((aligned(16))) float smem[(ONE ? 1 : 2) * SLAB];
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int n0 = blockIdx.x * T, m0 = blockIdx.y * T;
@@ -63,7 +66,7 @@ __global__ void __launch_bounds__(256, 2) gemm_tile_kernel(GemmParams p) {
     OpB ob;
     ob.init(p.B, p.ldb, n0, p.N, 0, p.K, p.K);
     float cs = 0.0f;
-    slab_pipeline(
+    slab_pipeline<ONE>(
         (p.K + KS - 1) / KS, [&](int t, auto st) { ob.load(t, sb[decltype(st)::value]); },
         [&](int t, auto st, auto buf, auto last) {
           ob.template store<decltype(last)::value>(t, sb[decltype(st)::value], smem + decltype(buf)::value * SLAB);
@@ -139,7 +142,7 @@ __global__ void __launch_bounds__(256, 2) gemm_tile_kernel(GemmParams p) {
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  slab_pipeline(
+  slab_pipeline<ONE>(
       n,
       [&](int t, auto st) {
         oa.load(t, sa[decltype(st)::value]);
@@ -159,7 +162,7 @@ __global__ void __launch_bounds__(256, 2) gemm_tile_kernel(GemmParams p) {
         mid();
         mfma(fa[0], fb[0]);
         if constexpr (decltype(full)::value) interleave(std::true_type{});
-        if (more) {
+        if (!ONE && more) {
           __syncthreads();
           frags(smem + (P ^ 1) * SLAB, 0, fa[0], fb[0]);
         }

@@ -370,7 +370,7 @@ __global__ void __launch_bounds__(256) rowreduce_kernel(const float* __restrict_
     }
     return a;
   };
-  slab_pipeline(
+  slab_pipeline<false>(
       (cols + Op::KS - 1) / Op::KS, [&](int t, auto s) { op.load(t, st[decltype(s)::value]); },
       [&](int t, auto s, auto buf, auto last) {
         op.template store<decltype(last)::value>(t, st[decltype(s)::value], smem[decltype(buf)::value], init);

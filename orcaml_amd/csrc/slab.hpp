@@ -150,12 +150,21 @@ struct TileOperand {
 // The loop's own slabs are never the last ones: their stores go unchecked, and every
 // load in it is unconditional (a load behind a branch would make the next store wait
 // for every load in flight).
-template <class Load, class Store, class Begin, class Use>
+// ONE: there is one slab (and one buffer).
+template <bool ONE, class Load, class Store, class Begin, class Use>
 __device__ __forceinline__ void slab_pipeline(int n, Load load, Store store, Begin begin, Use use) {
   constexpr std::integral_constant<int, 0> S0;
   constexpr std::integral_constant<int, 1> S1;
   constexpr std::false_type MID;
   constexpr std::true_type LAST;
+  if constexpr (ONE) {
+    load(0, S0);
+    store(0, S0, S0, LAST);
+    __syncthreads();
+    begin();
+    use(0, S0, []() {}, false, MID);
+    return;
+  }
   if (n > 2) {
     load(0, S0);
     load(1, S1);
