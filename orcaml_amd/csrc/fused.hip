@@ -181,36 +181,61 @@ __global__ void __launch_bounds__(256) softmax_ce_block_kernel(const float* __re
   }
 }
 
-// loss = (sum of row losses) * (1/B); correct = number of matching rows.
+// loss = (sum of row losses) * (1/B); correct = number of matching rows.  Thread t adds rows
+// t per .. t per + per - 1 in order, and the threads' sums go through a tree (t with t + 512,
+// then t + 256, ...).  One block, so its time is memory round trips and barriers: four rows per
+// load where a thread's rows come in fours, and the tree's last six levels, which stay in one
+// wave, without barriers (8192 rows: 10.4 -> 4.8 us).
 __global__ void __launch_bounds__(1024) ce_finish_kernel(const float* __restrict__ row_loss,
                                                           const int* __restrict__ row_correct, int B, float inv_b,
                                                           float* __restrict__ loss, int64_t* __restrict__ correct) {
   __shared__ float ls[1024];
-  __shared__ long long cs[1024];
+  __shared__ int cs[1024];
   const int t = threadIdx.x;
   const int per = (B + 1023) / 1024;
+  const int r0 = t * per, r1 = min(B, r0 + per);
   float s = 0.0f;
-  long long c = 0;
-  for (int k = 0; k < per; ++k) {
-    int r = t * per + k;
-    if (r < B) {
-      s = s + row_loss[r];
-      if (row_correct) c += row_correct[r];
+  int c = 0;
+  int r = r0;
+  if (per % 4 == 0 && ((reinterpret_cast<uintptr_t>(row_loss) | reinterpret_cast<uintptr_t>(row_correct)) & 15) == 0) {
+#pragma unroll 4
+    for (; r + 4 <= r1; r += 4) {
+      const floatx4 v = *reinterpret_cast<const floatx4*>(row_loss + r);
+      s = s + v.x;
+      s = s + v.y;
+      s = s + v.z;
+      s = s + v.w;
+      if (row_correct) {
+        const int4 w = *reinterpret_cast<const int4*>(row_correct + r);
+        c += (w.x + w.y) + (w.z + w.w);
+      }
     }
+  }
+  for (; r < r1; ++r) {
+    s = s + row_loss[r];
+    if (row_correct) c += row_correct[r];
   }
   ls[t] = s;
   cs[t] = c;
   __syncthreads();
-  for (int w = 512; w > 0; w >>= 1) {
+  for (int w = 512; w >= 64; w >>= 1) {
     if (t < w) {
-      ls[t] = ls[t] + ls[t + w];
-      cs[t] += cs[t + w];
+      s = s + ls[t + w];
+      c += cs[t + w];
+      ls[t] = s;
+      cs[t] = c;
     }
     __syncthreads();
   }
+  if (t >= 64) return;
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) {
+    s = s + __shfl_down(s, w);  // lanes from w on end with values nobody uses
+    c += __shfl_down(c, w);
+  }
   if (t == 0) {
-    if (loss) *loss = ls[0] * inv_b;
-    if (correct) *correct = cs[0];
+    if (loss) *loss = s * inv_b;
+    if (correct) *correct = c;
   }
 }
 
