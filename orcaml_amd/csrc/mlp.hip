@@ -529,9 +529,7 @@ static int read_arena(orca_hip_mlp* mlp, const float* arena, size_t index, float
     checked(mlp);
     check_index(mlp, index, n);
     if (!arena) fail(ORCA_HIP_ERR_INTERNAL, "state not present for this optimizer");
-    ORCA_HIP_CHECK(hipMemcpyAsync(host, arena + mlp->off[index], n * sizeof(float), hipMemcpyDeviceToHost,
-                                  mlp->ctx->stream));
-    host_sync(mlp->ctx);
+    read_host(mlp->ctx, host, arena + mlp->off[index], n * sizeof(float));
   });
 }
 
@@ -617,8 +615,7 @@ int orca_hip_mlp_get_logits(orca_hip_mlp* mlp, float* host, size_t n) {
     checked(mlp);
     size_t want = mlp->B * mlp->dims[mlp->L];
     if (n != want) fail(ORCA_HIP_ERR_SHAPE, "Shape mismatch during mlp_get_logits: expected " + std::to_string(want));
-    ORCA_HIP_CHECK(hipMemcpyAsync(host, mlp->logits, n * sizeof(float), hipMemcpyDeviceToHost, mlp->ctx->stream));
-    host_sync(mlp->ctx);
+    read_host(mlp->ctx, host, mlp->logits, n * sizeof(float));
   });
 }
 
@@ -638,8 +635,7 @@ int orca_hip_mlp_get_activation(orca_hip_mlp* mlp, size_t layer, float* host, si
     size_t want = mlp->B * mlp->dims[layer + 1];
     if (n != want) fail(ORCA_HIP_ERR_SHAPE, "Shape mismatch during mlp_get_activation: expected " + std::to_string(want));
     const float* src = layer + 1 < mlp->L ? mlp->H[layer] : mlp->logits;
-    ORCA_HIP_CHECK(hipMemcpyAsync(host, src, n * sizeof(float), hipMemcpyDeviceToHost, mlp->ctx->stream));
-    host_sync(mlp->ctx);
+    read_host(mlp->ctx, host, src, n * sizeof(float));
   });
 }
 

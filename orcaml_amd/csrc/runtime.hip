@@ -34,6 +34,23 @@ void upload_async(orca_hip_ctx* ctx, void* dst, const void* src, size_t bytes) {
   ctx->staging.upload(ctx, dst, src, bytes, ctx->stream);
 }
 
+void read_host(orca_hip_ctx* ctx, void* host, const void* device, size_t bytes) {
+  if (!bytes) return;
+  if (bytes >= StagingRing::kMinDownload) {
+    // pageable memory only: pinned memory takes the device's copy as it is
+    hipPointerAttribute_t at{};
+    const hipError_t e = hipPointerGetAttributes(&at, host);
+    if (e != hipSuccess) (void)hipGetLastError();
+    if (e != hipSuccess || at.type == hipMemoryTypeUnregistered) {
+      join_side(ctx);
+      ctx->staging.download(ctx, host, device, bytes, ctx->stream);
+      return;
+    }
+  }
+  ORCA_HIP_CHECK(hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, ctx->stream));
+  host_sync(ctx);
+}
+
 // ------------------------------------------------------------ small kernels
 __global__ void fill_kernel(float* __restrict__ dst, float v, size_t n) {
   size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -257,8 +274,7 @@ int orca_hip_d2h(orca_hip_ctx* ctx, void* dst, const void* src, size_t bytes) {
     if (!bytes) return;
     check_extent(ctx, src, bytes, "d2h");
     join_side(ctx);
-    ORCA_HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    host_sync(ctx);
+    read_host(ctx, dst, src, bytes);
   });
 }
 

@@ -150,10 +150,20 @@ class StagingRing {
  public:
   // Enqueues dst <- src (bytes) on `stream`; src may be reused on return.
   void upload(orca_hip_ctx* ctx, void* dst, const void* src, size_t bytes, hipStream_t stream);
+  // host <- device (bytes), waiting for it: parts go through the ring's slots, and helper
+  // threads that live as long as the call copy one part out while the device writes others.
+  // A plain copy to pageable memory takes turns instead (one part in, one part out on one
+  // thread), and the pages of a fresh destination are faulted in by that one thread.  80 MB
+  // into fresh memory: 7.5 -> 2.3 ms.
+  void download(orca_hip_ctx* ctx, void* host, const void* device, size_t bytes, hipStream_t stream);
   ~StagingRing();
 
   static constexpr size_t kCapacity = size_t(16) << 20;  // pinned bytes held per context
   static constexpr size_t kChunk = size_t(4) << 20;      // largest single region
+  // Reads from this size on go through download(); below it starting the helpers costs what
+  // they save (4 MiB: 0.25 ms as one copy, 0.37 ms in parts; 8 MiB: 0.49 and 0.37 ms).
+  static constexpr size_t kMinDownload = size_t(8) << 20;
+  static constexpr size_t kMaxHelpers = 6;
 
  private:
   struct Region {
@@ -336,6 +346,10 @@ void host_wait_event(orca_hip_ctx* ctx, hipEvent_t ev);
 // payloads travel as a kernel argument, larger ones through the staging ring.
 // The host buffer may be reused as soon as this returns.
 void upload_async(orca_hip_ctx* ctx, void* dst, const void* src, size_t bytes);
+
+// Host copy of device memory, complete on return (stream-ordered after the context stream's
+// work so far); counts its host waits.
+void read_host(orca_hip_ctx* ctx, void* host, const void* device, size_t bytes);
 
 // Allocates a fresh output buffer of n floats for a trait op.
 float* new_output(orca_hip_ctx* ctx, size_t n);

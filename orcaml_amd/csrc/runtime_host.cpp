@@ -5,10 +5,12 @@
 // plain C++ compiler against a HIP API stand-in for the sanitizer test
 // (tests/native).
 #include <algorithm>
+#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <sstream>
+#include <thread>
 
 #include "runtime.hpp"
 
@@ -382,6 +384,124 @@ void StagingRing::upload(orca_hip_ctx* ctx, void* dst, const void* src, size_t b
     d += part;
     h += part;
     bytes -= part;
+  }
+}
+
+namespace {
+// The host side of one download: parts whose device copy has arrived, and the threads that
+// copy them out.
+class PartCopier {
+ public:
+  PartCopier(char* host, const char* slots, size_t part, size_t n_slots, size_t bytes, size_t helpers)
+      : host_(host), slots_(slots), part_(part), n_slots_(n_slots), bytes_(bytes), done_((bytes + part - 1) / part) {
+    threads_.reserve(helpers);
+    for (size_t i = 0; i < helpers; ++i) {
+      try {
+        threads_.emplace_back([this] { run(); });
+      } catch (...) {
+        break;  // no more threads to be had: the others, or the caller, copy
+      }
+    }
+  }
+  ~PartCopier() {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      stop_ = true;
+    }
+    ready_cv_.notify_all();
+    for (auto& t : threads_) t.join();
+  }
+  // Part c is in its slot.
+  void ready(size_t c) {
+    if (threads_.empty()) {
+      copy(c);
+      done_[c] = true;
+      return;
+    }
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      ready_.push_back(c);
+    }
+    ready_cv_.notify_one();
+  }
+  bool done(size_t c) {
+    std::lock_guard<std::mutex> lk(mu_);
+    return done_[c];
+  }
+  void wait(size_t c) {
+    std::unique_lock<std::mutex> lk(mu_);
+    done_cv_.wait(lk, [&] { return done_[c]; });
+  }
+
+ private:
+  void copy(size_t c) {
+    std::memcpy(host_ + c * part_, slots_ + c % n_slots_ * part_, std::min(part_, bytes_ - c * part_));
+  }
+  void run() {
+    std::unique_lock<std::mutex> lk(mu_);
+    for (;;) {
+      ready_cv_.wait(lk, [&] { return stop_ || !ready_.empty(); });
+      if (ready_.empty()) return;
+      const size_t c = ready_.front();
+      ready_.pop_front();
+      lk.unlock();
+      copy(c);
+      lk.lock();
+      done_[c] = true;
+      done_cv_.notify_all();
+    }
+  }
+  char* host_;
+  const char* slots_;
+  const size_t part_, n_slots_, bytes_;
+  std::mutex mu_;
+  std::condition_variable ready_cv_, done_cv_;
+  std::deque<size_t> ready_;
+  std::vector<bool> done_;
+  bool stop_ = false;
+  std::vector<std::thread> threads_;
+};
+}  // namespace
+
+void StagingRing::download(orca_hip_ctx* ctx, void* host, const void* device, size_t bytes, hipStream_t stream) {
+  if (!bytes) return;
+  std::lock_guard<std::mutex> lk(mu_);
+  if (!base_) ORCA_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&base_), kCapacity, hipHostMallocDefault));
+  while (!inflight_.empty()) {  // uploads still reading the ring
+    host_wait_event(ctx, inflight_.front().done);
+    spare_.push_back(inflight_.front().done);
+    inflight_.pop_front();
+  }
+  head_ = 0;
+  // parts small enough that ten of them overlap, large enough to cost few hand-overs
+  const size_t part = bytes < (size_t(32) << 20) ? size_t(1) << 20 : size_t(2) << 20;
+  const size_t n = (bytes + part - 1) / part, n_slots = std::min(n, kCapacity / part);
+  while (spare_.size() < n_slots) {
+    hipEvent_t ev;
+    ORCA_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    spare_.push_back(ev);
+  }
+  const size_t helpers = std::min({n, kMaxHelpers, std::max<size_t>(1, std::thread::hardware_concurrency() / 2)});
+  PartCopier out(static_cast<char*>(host), base_, part, n_slots, bytes, helpers);
+  size_t issued = 0;
+  try {
+    for (size_t c = 0; c < n; ++c) {
+      // Every free slot gets its part; with none in flight the oldest part's copy is waited for.
+      while (issued < n && (issued < n_slots || issued <= c || out.done(issued - n_slots))) {
+        if (issued >= n_slots) out.wait(issued - n_slots);
+        const size_t slot = issued % n_slots;
+        ORCA_HIP_CHECK(hipMemcpyAsync(base_ + slot * part, static_cast<const char*>(device) + issued * part,
+                                      std::min(part, bytes - issued * part), hipMemcpyDeviceToHost, stream));
+        ORCA_HIP_CHECK(hipEventRecord(spare_[slot], stream));
+        ++issued;
+      }
+      host_wait_event(ctx, spare_[c % n_slots]);
+      out.ready(c);
+    }
+    for (size_t c = n > n_slots ? n - n_slots : 0; c < n; ++c) out.wait(c);
+  } catch (...) {
+    (void)hipStreamSynchronize(stream);  // nothing may write the ring after this call
+    throw;
   }
 }
 
