@@ -1433,6 +1433,7 @@ struct GemmPlan {
   int narrow;   // 0, or a narrow product: 1 NN (N <= 16), 2 NT (K <= 16), 3 TN (N <= 16)
   size_t BM, BN, mt, nt;
   int splits, k_chunk;  // for a narrow TN product: K slices and rows per slice
+  double us;            // choose_tile's estimate (0: it was not asked)
 };
 
 // Profiler names: "gemm_<op(A)><op(B)>", with "_pipe" on 16-byte aligned operands, "_skinny"
@@ -1461,23 +1462,26 @@ std::string kernel_name(const GemmPlan& g, bool ta, bool tb, size_t M, size_t cu
 // from about 230 tiles of 128 on nothing beats those (2048^3: 123 us, tiles of 64: 137).
 // A split's chunks are even runs of slabs; only splits that fill the CUs once or twice
 // are tried.
-void choose_tile(orca_hip_ctx* ctx, GemmPlan& g, bool trans_a, bool trans_b, size_t M, size_t N, size_t K,
-                 size_t batch) {
-  struct Form {
-    int tile;
-    size_t slab_k;
-    double block_us;
-    double slab_us[2][3];  // [unaligned operands][row-major operands: NT; NN, TT; TN]
-  };
-  static constexpr Form forms[4] = {{16, 256, 0.4, {{0.50, 0.60, 0.95}, {0.55, 0.70, 1.05}}},
+struct TileForm {
+  int tile;
+  size_t slab_k;
+  double block_us;
+  double slab_us[2][3];  // [unaligned operands][row-major operands: NT; NN, TT; TN]
+};
+constexpr TileForm kTileForms[4] = {{16, 256, 0.4, {{0.50, 0.60, 0.95}, {0.55, 0.70, 1.05}}},
                                     {32, 128, 0.5, {{0.64, 0.68, 0.85}, {0.68, 0.90, 0.95}}},
                                     {64, 64, 1.0, {{1.06, 1.06, 1.06}, {1.06, 1.10, 1.15}}},
                                     {128, BK, 3.0, {{1.82, 1.82, 1.82}, {1.84, 1.84, 1.84}}}};
+// The chain of adds of a column sum beside small tiles, us for k rows.
+constexpr double colsum_chain_us(size_t k) { return 4.0 + 0.0105 * (double)k; }
+
+void choose_tile(orca_hip_ctx* ctx, GemmPlan& g, bool trans_a, bool trans_b, size_t M, size_t N, size_t K,
+                 size_t batch) {
   const size_t target = (size_t)ctx->num_cus;
   const int mn_fast = (trans_a ? 1 : 0) + (trans_b ? 0 : 1);
   double best = 1e300;
   size_t best_chunk = K;
-  for (const Form& f : forms) {
+  for (const TileForm& f : kTileForms) {
     if (ctx->gemm_tile_bn && ctx->gemm_tile_bn != f.tile) continue;
     const size_t t = (size_t)f.tile;
     const size_t tiles = ((M + t - 1) / t) * ((N + t - 1) / t) * batch, slabs = (K + f.slab_k - 1) / f.slab_k;
@@ -1492,7 +1496,7 @@ void choose_tile(orca_hip_ctx* ctx, GemmPlan& g, bool trans_a, bool trans_b, siz
       double us = 3.0 + rounds * (f.block_us - (slabs == 1 && f.tile < 128 ? 0.15 : 0.0) + (double)per * f.slab_us[g.ua ? 1 : 0][mn_fast]);
       if (s > 1) us += 2.4 + (double)(s + 1) * (double)(batch * M * N) * 4.0 / 5e6;
       if (mn_fast == 2 && batch == 1) {
-        if (f.tile < 128) us = std::max(us, 4.0 + 0.0105 * (double)K);
+        if (f.tile < 128) us = std::max(us, colsum_chain_us(K));
         else us += s > 1 ? 4.0 + 0.009 * (double)K : 0.19 * (double)slabs;
       }
       if (us < best) {
@@ -1505,6 +1509,7 @@ void choose_tile(orca_hip_ctx* ctx, GemmPlan& g, bool trans_a, bool trans_b, siz
   }
   g.fast = !g.tile;
   g.k_chunk = (int)(g.splits > 1 ? best_chunk : K);
+  g.us = best;
 }
 
 GemmPlan plan_gemm(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t N, size_t K, const float* A,
@@ -1754,6 +1759,91 @@ bool narrow_linear_backward(orca_hip_ctx* ctx, const float* H, size_t B, size_t 
 }
 
 }  // namespace
+
+// dX = (dY W^T) masked and dW = X^T dY (+ column sums) in one launch, when the estimate says
+// that pays: the pair's time is its blocks' work spread over the CUs plus half a block's (or
+// one block's, if they all start at once), against the two plans' own times and the gap
+// between two launches.  784-1024-1024-10, 256 rows: 9.9 + 9.1 -> 15.3 us.  False (nothing
+// launched) when the two run apart.
+bool gemm_linear_backward(orca_hip_ctx* ctx, size_t B, size_t K, size_t N, const float* X, const float* dY,
+                          const float* W, const float* mask, float* dX, float* dW, float* colsum) {
+  if (!B || !K || !N || B > INT32_MAX || K > INT32_MAX || N > INT32_MAX || ctx->gemm_tile_bn || ctx->gemm_splits) return false;
+  const GemmPlan px = plan_gemm(ctx, false, true, B, K, N, dY, N, 0, W, N, 0, 1, ORCA_HIP_EPI_RELU_MASK);
+  const GemmPlan pw = plan_gemm(ctx, true, false, K, N, B, X, K, 0, dY, N, 0, 1);
+  if (px.us == 0.0 || pw.us == 0.0) return false;  // narrow, banded or generic
+  const int ua = px.ua || pw.ua ? 1 : 0;
+  struct Pair {
+    int x, w;
+  };
+  static constexpr Pair pairs[5] = {{0, 0}, {1, 0}, {1, 1}, {1, 2}, {2, 2}};  // of kTileForms
+  const double cus = (double)ctx->num_cus;
+  auto tiles = [](size_t m, size_t n, size_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
+  auto block = [&](const TileForm& f, int mn_fast, size_t k) {
+    return f.block_us + (double)((k + f.slab_k - 1) / f.slab_k) * f.slab_us[ua][mn_fast];
+  };
+  int best = -1;
+  double best_us = px.us + pw.us + 1.0;
+  for (int i = 0; i < 5; ++i) {
+    const TileForm &fx = kTileForms[pairs[i].x], &fw = kTileForms[pairs[i].w];
+    const double bx = block(fx, 0, N), bw = block(fw, 2, B);
+    const double nx = (double)tiles(B, K, (size_t)fx.tile), nw = (double)tiles(K, N, (size_t)fw.tile);
+    const double longest = std::max(bx, bw), spread = (nx * bx + nw * bw) / cus + 0.5 * longest;
+    const double us = std::max(3.0 + (nx + nw <= cus ? longest : std::max(longest, spread)), colsum ? colsum_chain_us(B) : 0.0);
+    if (us < best_us) {
+      best_us = us;
+      best = i;
+    }
+  }
+  if (best < 0) return false;
+  const int tx = kTileForms[pairs[best].x].tile, tw = kTileForms[pairs[best].w].tile;
+  GemmParams x{}, w{};
+  x.A = dY;
+  x.B = W;
+  x.C = dX;
+  x.lda = x.ldb = (int64_t)N;
+  x.ldc = x.ldmask = (int64_t)K;
+  x.M = (int)B;
+  x.N = (int)K;
+  x.K = x.k_chunk = (int)N;
+  x.splits = 1;
+  x.epi = ORCA_HIP_EPI_RELU_MASK;
+  x.mask = mask;
+  w.A = X;
+  w.B = dY;
+  w.C = dW;
+  w.lda = (int64_t)K;
+  w.ldb = w.ldc = (int64_t)N;
+  w.M = (int)K;
+  w.N = (int)N;
+  w.K = w.k_chunk = (int)B;
+  w.splits = 1;
+  w.epi = ORCA_HIP_EPI_NONE;
+  w.colsum = colsum;
+  const size_t x_nt = (K + tx - 1) / tx, x_blocks = x_nt * ((B + tx - 1) / tx);
+  const size_t w_nt = (N + tw - 1) / tw, w_sums = colsum ? w_nt : 0, w_blocks = w_nt * ((K + tw - 1) / tw) + w_sums;
+  if (x_blocks + w_blocks > INT32_MAX) return false;
+  std::string pname;
+  if (ctx->prof.enabled)
+    pname = "gemm_linear_bw " + std::to_string(B) + "x" + std::to_string(K) + "x" + std::to_string(N);
+  ProfScope ps(ctx, pname.c_str(), 4.0 * (double)B * K * N, 4.0 * (double)(2 * B * N + 2 * K * N + 3 * B * K));
+#define PAIR_LAUNCH(TX_, TW_)                                                                                        \
+  do {                                                                                                               \
+    if (ua)                                                                                                          \
+      hipLaunchKernelGGL((gemm_tile_pair_kernel<TX_, TW_, true>), dim3((unsigned)(x_blocks + w_blocks)), dim3(256), 0, \
+                         ctx->stream, x, w, (int)w_sums, (int)x_blocks, (int)x_nt, (int)w_nt);                       \
+    else                                                                                                             \
+      hipLaunchKernelGGL((gemm_tile_pair_kernel<TX_, TW_, false>), dim3((unsigned)(x_blocks + w_blocks)), dim3(256), \
+                         0, ctx->stream, x, w, (int)w_sums, (int)x_blocks, (int)x_nt, (int)w_nt);                    \
+  } while (0)
+  if (tx == 16) PAIR_LAUNCH(16, 16);
+  else if (tx == 32 && tw == 16) PAIR_LAUNCH(32, 16);
+  else if (tx == 32 && tw == 32) PAIR_LAUNCH(32, 32);
+  else if (tx == 32) PAIR_LAUNCH(32, 64);
+  else PAIR_LAUNCH(64, 64);
+#undef PAIR_LAUNCH
+  ORCA_HIP_CHECK(hipGetLastError());
+  return true;
+}
 
 size_t gemm_workspace_floats(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t N, size_t K,
                              const float* A, size_t lda, size_t sa, const float* B, size_t ldb, size_t sb,

@@ -46,19 +46,22 @@ __device__ __forceinline__ void tile_store_one(const GemmParams& p, float* C, in
 // ONE: K is at most one slab.  Without the loop and its second buffer four blocks fit a CU
 // instead of two, so that some load or store while others multiply, and the code is a
 // third as long.
+template <int T, bool TA, bool TB, bool UA>
+constexpr int tile_slab_floats() {
+  return TileOperand<T, !TA, UA>::FLOATS + TileOperand<T, TB, UA>::FLOATS;
+}
+
 template <int T, bool TA, bool TB, bool UA, bool ONE>
-__global__ void __launch_bounds__(256, ONE ? 4 : 2) gemm_tile_kernel(GemmParams p) {
+__device__ __forceinline__ void tile_product(const GemmParams& p, int bx, int by, int bz, float* __restrict__ smem) {
   using OpA = TileOperand<T, !TA, UA>;
   using OpB = TileOperand<T, TB, UA>;
   constexpr int KS = OpA::KS;
-  constexpr int RED = T == 64 ? 0 : 4 * T * T;
-  constexpr int SLAB = OpA::FLOATS + OpB::FLOATS;
-  static_assert(SLAB >= RED, "the waves' blocks fit a slab buffer");
-  __shared__ __attribute__((aligned(16))) float smem[(ONE ? 1 : 2) * SLAB];
+  constexpr int SLAB = tile_slab_floats<T, TA, TB, UA>();
+  static_assert(SLAB >= (T == 64 ? 0 : 4 * T * T), "the waves' blocks fit a slab buffer");
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int n0 = blockIdx.x * T, m0 = blockIdx.y * T;
-  const int bz = blockIdx.z, batch = bz / p.splits, split = bz % p.splits;
+  const int n0 = bx * T, m0 = by * T;
+  const int batch = bz / p.splits, split = bz % p.splits;
   floatx4 sa[2][4], sb[2][4];  // the register stages
 
   if (!TB && m0 >= p.M) {  // the column sums
@@ -197,5 +200,31 @@ __global__ void __launch_bounds__(256, ONE ? 4 : 2) gemm_tile_kernel(GemmParams 
       const float v = ((smem[o] + smem[o + T * T]) + smem[o + 2 * T * T]) + smem[o + 3 * T * T];
       if (row < p.M && col < p.N) tile_store_one(p, C, ldc, epi, row, col, v);
     }
+  }
+}
+
+template <int T, bool TA, bool TB, bool UA, bool ONE>
+__global__ void __launch_bounds__(256, ONE ? 4 : 2) gemm_tile_kernel(GemmParams p) {
+  __shared__ __attribute__((aligned(16))) float smem[(ONE ? 1 : 2) * tile_slab_floats<T, TA, TB, UA>()];
+  // the column sums' chain of adds starts first
+  const int by = TB || !p.colsum ? blockIdx.y : blockIdx.y ? blockIdx.y - 1 : (p.M + T - 1) / T;
+  tile_product<T, TA, TB, UA, ONE>(p, blockIdx.x, by, blockIdx.z, smem);
+}
+
+// A Linear layer's two backward products from one grid: the column sums of dW = X^T dY (w;
+// w_sums blocks, none without them), dX = dY W^T (x; x_blocks, x_nt of them per row of tiles)
+// and dW itself.  Neither
+// fills the GPU at the sizes that come here, and each launch of its own pays the start and
+// the drain of a grid again.
+template <int TX, int TW, bool UA>
+__global__ void __launch_bounds__(256, 2) gemm_tile_pair_kernel(GemmParams x, GemmParams w, int w_sums, int x_blocks, int x_nt, int w_nt) {
+  constexpr int SX = tile_slab_floats<TX, false, true, UA>(), SW = tile_slab_floats<TW, true, false, UA>();
+  __shared__ __attribute__((aligned(16))) float smem[2 * (SX > SW ? SX : SW)];
+  const int b = (int)blockIdx.x - w_sums, c = b - x_blocks;
+  if (b >= 0 && c < 0) {
+    tile_product<TX, false, true, UA, false>(x, b % x_nt, b / x_nt, 0, smem);
+  } else {
+    const int by = b < 0 ? (w.M + TW - 1) / TW : c / w_nt;
+    tile_product<TW, true, false, UA, false>(w, b < 0 ? (int)blockIdx.x : c % w_nt, by, 0, smem);
   }
 }

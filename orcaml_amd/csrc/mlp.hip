@@ -235,6 +235,15 @@ void step_body(orca_hip_mlp* m, const AdamWScalars* kdev) {
     ew.ws_floats = m->gemm_ws_floats;
     // bias gradient (the head's backward kernel already summed the layer below it)
     ew.colsum = m->head_db && l + 2 == L ? nullptr : m->G + m->off[2 * l + 1];
+    // Small layers: both products from one grid (a model with a second stream keeps them
+    // apart, for the update that starts between them).
+    if (l > 0 && !m->side &&
+        gemm_linear_backward(ctx, B, K, N, a, g, m->P + m->off[2 * l], m->H[l - 1], m->dz[ping], m->G + m->off[2 * l],
+                             ew.colsum)) {
+      g = m->dz[ping];
+      ping ^= 1;
+      continue;
+    }
     // Layers >= 1 have all their gradients after dW of layer 1; with a second
     // arena nothing of this step writes the P that layer 1's dZ reads.
     const bool early = l == 1 && m->P_next && overlap;

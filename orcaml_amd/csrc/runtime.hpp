@@ -393,6 +393,12 @@ void gemm(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t N, siz
           size_t lda, size_t sa, const float* B, size_t ldb, size_t sb, float* C, size_t ldc, size_t sc,
           size_t batch, const GemmEpi& epi);
 
+// A hidden Linear's backward in one launch where that pays (false: nothing done, run the two
+// products): dX[B][K] = (dY[B][N] W[K][N]^T) * [mask[B][K] > 0], dW[K][N] = X[B][K]^T dY and,
+// when colsum is set, the bias gradient in ascending row order.
+bool gemm_linear_backward(orca_hip_ctx* ctx, size_t B, size_t K, size_t N, const float* X, const float* dY,
+                          const float* W, const float* mask, float* dX, float* dW, float* colsum);
+
 // row_loss / row_correct: optional caller-owned [B] workspaces (else from the context cache).
 void softmax_ce(orca_hip_ctx* ctx, const float* logits, size_t B, size_t C, const float* onehot,
                 const int32_t* labels, float* loss, float* dlogits, int32_t* preds, int64_t* correct,
