@@ -14,6 +14,7 @@
 
 #include "ce_row.hpp"
 #include "runtime.hpp"
+#include "slab.hpp"
 
 namespace orca_hip {
 // Fixed device scratch of orca_hip_relu_bw_colsum_noalloc: 2^20 floats (4 MiB)
@@ -28,8 +29,6 @@ static __device__ __align__(256) float scratch[orca_hip::kStaticScratchFloats];
 
 namespace orca_hip {
 namespace {
-
-typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // One wave per row.  Logits stay in registers, VPL values per lane: column
 // c = lane + 64 j (scalar loads), or, when VEC (C a multiple of 4 and 16-byte
@@ -242,51 +241,73 @@ __global__ void __launch_bounds__(1024) ce_finish_kernel(const float* __restrict
 constexpr int kRowsPerChunk = 64;  // rows per column-sum partial of the ReLU-backward kernels
 
 // dpre = pre > 0 ? g : 0 and per-chunk column partial sums (4 columns per
-// thread).  Rows go RB_UNROLL at a time, all loads issued before any use;
-// g and pre are read with ordinary loads, dpre is written with non-temporal
-// stores ([8192, 4096]: 62.0 us against 67.8 with non-temporal loads too,
-// 77.1 with ordinary stores too).
-constexpr int RB_UNROLL = 8;
+// thread).  Rows go U at a time, all loads issued before any use; g and pre are
+// read with ordinary loads, dpre is written with non-temporal stores ([8192,
+// 4096]: 62.0 us against 67.8 with non-temporal loads too, 77.1 with ordinary
+// stores too).  U is 8 where the grid fills the GPU and 16 where a chunk's chain
+// of round trips is the time ([200, 333]: 18.7 -> 11.1 us a call).  UA: any column count
+// and alignment, the same 16-byte accesses at 4-byte addresses; the thread of a
+// row's last one to three columns loads the row's last four and stores its own
+// ([1160, 2133]: 31.5 -> 12.8 us, [8190, 4095]: 103 -> 68).
+constexpr int RB_UNROLL = 8, RB_UNROLL_SMALL = 16;
 
-__global__ void __launch_bounds__(256) relu_bw_colsum_vec_kernel(const float4* __restrict__ g, const float4* __restrict__ pre,
-                                                                 size_t rows, size_t cols4, int rows_per_chunk,
-                                                                 float4* __restrict__ dpre, float4* __restrict__ partial) {
-  size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols4) return;
-  size_t r0 = (size_t)blockIdx.y * rows_per_chunk;
-  size_t r1 = r0 + rows_per_chunk < rows ? r0 + rows_per_chunk : rows;
-  const floatx4* gv = reinterpret_cast<const floatx4*>(g);
-  const floatx4* pv = reinterpret_cast<const floatx4*>(pre);
-  floatx4* dv = reinterpret_cast<floatx4*>(dpre);
-  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (size_t rb = r0; rb < r1; rb += RB_UNROLL) {
-    floatx4 ga[RB_UNROLL], pa[RB_UNROLL];
+template <bool UA, int U>
+__global__ void __launch_bounds__(256) relu_bw_colsum_kernel(const float* __restrict__ g, const float* __restrict__ pre,
+                                                             size_t rows, size_t cols, int rows_per_chunk,
+                                                             float* __restrict__ dpre, float* __restrict__ partial) {
+  using vec = typename std::conditional<UA, floatx4_u, floatx4>::type;
+  const size_t c = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (c >= cols) return;
+  const size_t cl = UA && c + 4 > cols ? cols - 4 : c;  // where this thread's four columns start
+  const int own = (int)(c - cl);                        // the first of them that it stores
+  const size_t r0 = (size_t)blockIdx.y * rows_per_chunk;
+  const size_t r1 = r0 + rows_per_chunk < rows ? r0 + rows_per_chunk : rows;
+  floatx4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+  // U rows; `tail`: fewer than U are left, the others are loaded again (no branch around a
+  // load) and not used.
+  auto group = [&](size_t rb, auto tail) {
+    floatx4 ga[U], pa[U];
 #pragma unroll
-    for (int u = 0; u < RB_UNROLL; ++u) {
-      const size_t r = rb + u;
-      if (r < r1) {
-        ga[u] = gv[r * cols4 + c];
-        pa[u] = pv[r * cols4 + c];
-      }
+    for (int u = 0; u < U; ++u) {
+      const size_t r = decltype(tail)::value && rb + u >= r1 ? r1 - 1 : rb + u;
+      ga[u] = *reinterpret_cast<const vec*>(g + r * cols + cl);
+      pa[u] = *reinterpret_cast<const vec*>(pre + r * cols + cl);
     }
 #pragma unroll
-    for (int u = 0; u < RB_UNROLL; ++u) {
-      const size_t r = rb + u;
-      if (r < r1) {
-        const floatx4 gg = ga[u], pp = pa[u];
-        const floatx4 d = {pp.x > 0.0f ? gg.x : 0.0f, pp.y > 0.0f ? gg.y : 0.0f, pp.z > 0.0f ? gg.z : 0.0f,
-                           pp.w > 0.0f ? gg.w : 0.0f};
-        __builtin_nontemporal_store(d, dv + r * cols4 + c);
-        s.x = s.x + d.x;
-        s.y = s.y + d.y;
-        s.z = s.z + d.z;
-        s.w = s.w + d.w;
+    for (int u = 0; u < U; ++u) {
+      if (decltype(tail)::value && rb + u >= r1) break;
+      const floatx4 gg = ga[u], pp = pa[u];
+      const floatx4 d = {pp.x > 0.0f ? gg.x : 0.0f, pp.y > 0.0f ? gg.y : 0.0f, pp.z > 0.0f ? gg.z : 0.0f,
+                         pp.w > 0.0f ? gg.w : 0.0f};
+      float* out = dpre + (rb + u) * cols + cl;
+      if (!UA || own == 0) {
+        __builtin_nontemporal_store((vec)d, reinterpret_cast<vec*>(out));
+      } else {
+        if (own <= 1) out[1] = d.y;
+        if (own <= 2) out[2] = d.z;
+        out[3] = d.w;
       }
+      s.x = s.x + d.x;
+      s.y = s.y + d.y;
+      s.z = s.z + d.z;
+      s.w = s.w + d.w;
     }
+  };
+  size_t rb = r0;
+  for (; rb + U <= r1; rb += U) group(rb, std::false_type{});
+  if (rb < r1) group(rb, std::true_type{});
+  if (!partial) return;
+  float* out = partial + (size_t)blockIdx.y * cols + cl;
+  if (!UA || own == 0) {
+    *reinterpret_cast<vec*>(out) = s;
+  } else {
+    if (own <= 1) out[1] = s.y;
+    if (own <= 2) out[2] = s.z;
+    out[3] = s.w;
   }
-  if (partial) partial[(size_t)blockIdx.y * cols4 + c] = s;
 }
 
+// Fewer than four columns.
 __global__ void __launch_bounds__(256) relu_bw_colsum_scalar_kernel(const float* __restrict__ g, const float* __restrict__ pre,
                                                                     size_t rows, size_t cols, int rows_per_chunk,
                                                                     float* __restrict__ dpre, float* __restrict__ partial) {
@@ -439,9 +460,10 @@ __global__ void adamw_store_scalars_kernel(AdamWScalars* dst, AdamWScalars s) { 
 // python/orca/optim/adamw.py:66-99 and sgd.py:46-79, as one pass): segment i
 // covers float4 groups [start4[i], start4[i + 1]) of the launch's index space
 // and ceil(n / 4) groups of its own arrays.  A thread finds its segment by
-// binary search over the (uniform) table; whole groups of 16-byte-aligned
-// segments take float4 accesses, the rest (a segment's last partial group,
-// unaligned segments) element by element.  Same per-element arithmetic as the
+// binary search over the (uniform) table; whole groups take 16-byte accesses
+// (UA, when some segment is not 16-byte aligned, at 4-byte addresses: parameters
+// packed without padding; 2^26 in six: 569 -> 333 us), a segment's last partial group
+// goes element by element.  Same per-element arithmetic as the
 // one-parameter kernels, so the same bits.
 constexpr int kOptSegs = ORCA_HIP_OPT_MAX_SEGMENTS;
 struct OptSegs {
@@ -452,7 +474,6 @@ struct OptSegs {
   float* v[kOptSegs];
   uint64_t n[kOptSegs];
   uint64_t start4[kOptSegs + 1];
-  uint32_t vec_mask;  // bit i: segment i's arrays are all 16-byte aligned
   int count;
 };
 
@@ -466,32 +487,34 @@ __device__ __forceinline__ int opt_segment(const OptSegs& s, uint64_t q) {
   return lo;
 }
 
-template <bool ADAMW>
+template <bool ADAMW, bool UA>
 __device__ __forceinline__ void opt_multi_group(const OptSegs& s, const AdamWScalars& k, float lr, uint64_t q) {
   const int i = opt_segment(s, q);
   const uint64_t e0 = 4 * (q - s.start4[i]);
   const uint64_t n = s.n[i];
-  if (((s.vec_mask >> i) & 1) && e0 + 4 <= n) {
-    const uint64_t j = e0 / 4;
-    const floatx4 pp = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(s.ps[i]) + j);
-    const floatx4 gg = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(s.g[i]) + j);
+  if (e0 + 4 <= n) {
+    using vec = typename std::conditional<UA, floatx4_u, floatx4>::type;
+    auto ld = [&](const float* a) -> floatx4 { return __builtin_nontemporal_load(reinterpret_cast<const vec*>(a + e0)); };
+    auto st = [&](floatx4 x, float* a) { __builtin_nontemporal_store((vec)x, reinterpret_cast<vec*>(a + e0)); };
+    const floatx4 pp = ld(s.ps[i]);
+    const floatx4 gg = ld(s.g[i]);
     if (ADAMW) {
-      const floatx4 mm = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(s.m[i]) + j);
-      const floatx4 vv = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(s.v[i]) + j);
+      const floatx4 mm = ld(s.m[i]);
+      const floatx4 vv = ld(s.v[i]);
       float pa[4] = {pp.x, pp.y, pp.z, pp.w}, ma[4] = {mm.x, mm.y, mm.z, mm.w}, va[4] = {vv.x, vv.y, vv.z, vv.w};
       const float ga[4] = {gg.x, gg.y, gg.z, gg.w};
 #pragma unroll
       for (int u = 0; u < 4; ++u) adamw_elem(pa[u], ga[u], ma[u], va[u], k);
-      __builtin_nontemporal_store(floatx4{pa[0], pa[1], pa[2], pa[3]}, reinterpret_cast<floatx4*>(s.pd[i]) + j);
-      __builtin_nontemporal_store(floatx4{ma[0], ma[1], ma[2], ma[3]}, reinterpret_cast<floatx4*>(s.m[i]) + j);
-      __builtin_nontemporal_store(floatx4{va[0], va[1], va[2], va[3]}, reinterpret_cast<floatx4*>(s.v[i]) + j);
+      st(floatx4{pa[0], pa[1], pa[2], pa[3]}, s.pd[i]);
+      st(floatx4{ma[0], ma[1], ma[2], ma[3]}, s.m[i]);
+      st(floatx4{va[0], va[1], va[2], va[3]}, s.v[i]);
     } else {
       floatx4 r;
       r.x = pp.x - gg.x * lr;
       r.y = pp.y - gg.y * lr;
       r.z = pp.z - gg.z * lr;
       r.w = pp.w - gg.w * lr;
-      __builtin_nontemporal_store(r, reinterpret_cast<floatx4*>(s.pd[i]) + j);
+      st(r, s.pd[i]);
     }
     return;
   }
@@ -510,10 +533,10 @@ __device__ __forceinline__ void opt_multi_group(const OptSegs& s, const AdamWSca
 
 // One float4 group per thread on the full grid; a bounded grid (a pass beside
 // other work) strides over the groups.
-template <bool ADAMW>
+template <bool ADAMW, bool UA>
 __global__ void __launch_bounds__(256) opt_multi_kernel(OptSegs s, AdamWScalars k, float lr) {
   const uint64_t total = s.start4[s.count], stride = (uint64_t)gridDim.x * 256;
-  for (uint64_t q = (uint64_t)blockIdx.x * 256 + threadIdx.x; q < total; q += stride) opt_multi_group<ADAMW>(s, k, lr, q);
+  for (uint64_t q = (uint64_t)blockIdx.x * 256 + threadIdx.x; q < total; q += stride) opt_multi_group<ADAMW, UA>(s, k, lr, q);
 }
 
 __global__ void __launch_bounds__(256) sgd_vec_kernel(float4* __restrict__ p, const float4* __restrict__ g, size_t n4, float lr) {
@@ -679,6 +702,7 @@ void opt_multi(orca_hip_ctx* ctx, const orca_hip_opt_segment* segs, size_t n_seg
     OptSegs t{};
     uint64_t total4 = 0;
     double bytes = 0.0;
+    bool vec = true;  // every segment's arrays are 16-byte aligned
     for (size_t i = b; i < n_segs && t.count < kOptSegs; ++i) {
       const orca_hip_opt_segment& sg = segs[i];
       const size_t nb = sg.n * sizeof(float);
@@ -700,9 +724,8 @@ void opt_multi(orca_hip_ctx* ctx, const orca_hip_opt_segment* segs, size_t n_seg
       t.n[c] = sg.n;
       t.start4[c] = total4;
       total4 += (sg.n + 3) / 4;
-      const bool vec = aligned16(sg.p_src) && aligned16(sg.p_dst) && aligned16(sg.g) &&
-                       (!adamw_ || (aligned16(sg.m) && aligned16(sg.v)));
-      if (vec) t.vec_mask |= 1u << c;
+      vec = vec && aligned16(sg.p_src) && aligned16(sg.p_dst) && aligned16(sg.g) &&
+            (!adamw_ || (aligned16(sg.m) && aligned16(sg.v)));
       bytes += (adamw_ ? 28.0 : 12.0) * (double)sg.n;
     }
     t.start4[t.count] = total4;
@@ -716,10 +739,13 @@ void opt_multi(orca_hip_ctx* ctx, const orca_hip_opt_segment* segs, size_t n_seg
     ProfScope ps(ctx, ctx->main ? (adamw_ ? "adamw_multi_overlapped" : "sgd_multi_overlapped")
                                 : (adamw_ ? "adamw_multi" : "sgd_multi"),
                  0.0, bytes);
-    if (adamw_)
-      hipLaunchKernelGGL(opt_multi_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, t, k, lr);
-    else
-      hipLaunchKernelGGL(opt_multi_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, t, k, lr);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, t, k, lr);
+    };
+    if (adamw_ && vec) launch(opt_multi_kernel<true, false>);
+    else if (adamw_) launch(opt_multi_kernel<true, true>);
+    else if (vec) launch(opt_multi_kernel<false, false>);
+    else launch(opt_multi_kernel<false, true>);
     ORCA_HIP_CHECK(hipGetLastError());
   }
 }
@@ -874,17 +900,17 @@ void relu_bw_colsum_launch(orca_hip_ctx* ctx, const float* grad, const float* pr
     const size_t chunks = (rows + rows_per_chunk - 1) / rows_per_chunk;
     {
       ProfScope ps(ctx, "relu_bw_colsum", 0.0, 12.0 * (double)rows * cols + (colsum ? 4.0 * cols : 0.0));
-      if (cols % 4 == 0 && aligned16(grad) && aligned16(pre) && aligned16(dpre)) {
-        size_t cols4 = cols / 4;
-        dim3 grid((unsigned)((cols4 + 255) / 256), (unsigned)chunks);
-        hipLaunchKernelGGL(relu_bw_colsum_vec_kernel, grid, dim3(256), 0, ctx->stream,
-                           reinterpret_cast<const float4*>(grad), reinterpret_cast<const float4*>(pre), rows, cols4,
-                           rows_per_chunk, reinterpret_cast<float4*>(dpre), reinterpret_cast<float4*>(part));
-      } else {
-        dim3 grid((unsigned)((cols + 255) / 256), (unsigned)chunks);
-        hipLaunchKernelGGL(relu_bw_colsum_scalar_kernel, grid, dim3(256), 0, ctx->stream, grad, pre, rows, cols,
-                           rows_per_chunk, dpre, part);
-      }
+      const dim3 grid((unsigned)(((cols + 3) / 4 + 255) / 256), (unsigned)chunks);
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, ctx->stream, grad, pre, rows, cols, rows_per_chunk, dpre, part);
+      };
+      const bool vec = cols % 4 == 0 && aligned16(grad) && aligned16(pre) && aligned16(dpre) && aligned16(part);
+      const bool small = (size_t)grid.x * grid.y <= 2 * (size_t)ctx->num_cus;
+      if (cols < 4) launch(relu_bw_colsum_scalar_kernel);
+      else if (vec && small) launch(relu_bw_colsum_kernel<false, RB_UNROLL_SMALL>);
+      else if (vec) launch(relu_bw_colsum_kernel<false, RB_UNROLL>);
+      else if (small) launch(relu_bw_colsum_kernel<true, RB_UNROLL_SMALL>);
+      else launch(relu_bw_colsum_kernel<true, RB_UNROLL>);
       ORCA_HIP_CHECK(hipGetLastError());
     }
     if (colsum) {
