@@ -1484,6 +1484,7 @@ void choose_tile(orca_hip_ctx* ctx, GemmPlan& g, bool trans_a, bool trans_b, siz
   for (const TileForm& f : kTileForms) {
     if (ctx->gemm_tile_bn && ctx->gemm_tile_bn != f.tile) continue;
     const size_t t = (size_t)f.tile;
+    if (f.tile < 128 && (M + t - 1) / t >= 65535) continue;  // grid rows (and one for column sums): 2^20 rows of 16
     const size_t tiles = ((M + t - 1) / t) * ((N + t - 1) / t) * batch, slabs = (K + f.slab_k - 1) / f.slab_k;
     for (int j = 0; j < 3; ++j) {
       size_t s = j == 0 ? 1 : std::min<size_t>(std::min<size_t>((size_t)j * target / tiles, slabs / 2), 64);

@@ -144,3 +144,12 @@ def test_every_tile_batched(tctx, batch, M, N, K):
             be.from_f32_slice((batch, N, K), Bt), (batch, N, K), 1, 2)
         got = be.to_f32_vec(be.matmul(a, b, (batch, M, K), (batch, K, N))).reshape(batch, M, N)
         np.testing.assert_array_equal(got, want)
+
+
+def test_more_rows_than_grid_rows_of_small_tiles(ctx):
+    """2^21 + 3 rows: 32-row tiles, the cheapest for this width, would need 65537 grid rows."""
+    rng = np.random.default_rng(5)
+    A, B = int_matrix(rng, ((1 << 21) + 3, 32), -2, 3), int_matrix(rng, (32, 20), -2, 3)
+    a, b, c = ctx.upload(A), ctx.upload(B), ctx.alloc(A.shape[0] * 80)
+    _lib.call("orca_hip_gemm", ctx.handle, 0, 0, A.shape[0], 20, 32, a.ptr, 32, b.ptr, 20, c.ptr, 20, None)
+    np.testing.assert_array_equal(c.download(count=A.shape[0] * 20).reshape(-1, 20), A @ B)
