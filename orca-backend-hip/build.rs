@@ -56,7 +56,7 @@ fn main() {
             .arg(&obj));
         objs.push(obj);
     }
-    for hdr in ["runtime.hpp", "ew_ops.hpp", "ce_row.hpp", "slab.hpp", "gemm_tile.hpp"].iter() {
+    for hdr in ["runtime.hpp", "ew_ops.hpp", "ce_row.hpp", "slab.hpp", "gemm_tile.hpp", "optim.hpp"].iter() {
         println!("cargo:rerun-if-changed={}", csrc.join(hdr).display());
     }
     println!("cargo:rerun-if-changed={}", Path::new(&pkg).join("../include/orca_hip.h").display());

@@ -13,6 +13,7 @@
 #include <mutex>
 
 #include "ce_row.hpp"
+#include "optim.hpp"
 #include "runtime.hpp"
 #include "slab.hpp"
 
@@ -357,19 +358,6 @@ __global__ void __launch_bounds__(256) chunk_reduce_kernel(const float* __restri
     for (int p = 1; p < CR_PARTS; ++p) t = t + q[p][lc];
     out[c] = t;
   }
-}
-
-__device__ __forceinline__ void adamw_elem(float& p, float g, float& m, float& v, const AdamWScalars& k) {
-  float d = p * k.decay;                // p * (1 - lr*wd)
-  float mn = (m * k.b1) + (g * k.omb1); // m*b1 + g*(1-b1)
-  float vn = (v * k.b2) + ((g * g) * k.omb2);
-  float mh = mn * k.c1;
-  float vh = vn * k.c2;
-  float den = sqrtf(vh) + k.eps;
-  float u = (mh / den) * k.lr;
-  p = d - u;
-  m = mn;
-  v = vn;
 }
 
 // One float4 of every array per thread, a flat grid, and non-temporal loads

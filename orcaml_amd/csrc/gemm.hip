@@ -29,6 +29,7 @@
 
 #include <hip/hip_ext.h>
 
+#include "optim.hpp"
 #include "runtime.hpp"
 #include "slab.hpp"
 
@@ -1842,6 +1843,59 @@ bool gemm_linear_backward(orca_hip_ctx* ctx, size_t B, size_t K, size_t N, const
   else if (tx == 32) PAIR_LAUNCH(32, 64);
   else PAIR_LAUNCH(64, 64);
 #undef PAIR_LAUNCH
+  ORCA_HIP_CHECK(hipGetLastError());
+  return true;
+}
+
+bool gemm_first_layer_update(orca_hip_ctx* ctx, size_t B, size_t K, size_t N, const float* X, const float* dY,
+                             bool bias_sum, size_t bias, size_t rest, const ArenaUpdate& u) {
+  if (!B || !K || !N || B > INT32_MAX || K > INT32_MAX || N > INT32_MAX) return false;
+  const GemmPlan plan = plan_gemm(ctx, true, false, K, N, B, X, K, 0, dY, N, 0, 1, ORCA_HIP_EPI_NONE, 1);
+  if (!plan.tile || plan.splits != 1) return false;  // narrow, banded, 128 x 128 tiles, generic or split
+  GemmParams w{};
+  w.A = X;
+  w.B = dY;
+  w.C = u.G;
+  w.lda = (int64_t)K;
+  w.ldb = w.ldc = (int64_t)N;
+  w.M = (int)K;
+  w.N = (int)N;
+  w.K = w.k_chunk = (int)B;
+  w.splits = 1;
+  w.epi = ORCA_HIP_EPI_NONE;
+  w.colsum = bias_sum ? u.G + bias : nullptr;
+  const size_t r0 = bias_sum ? rest : bias;  // a bias whose gradient is there already goes with the rest
+  const size_t sums = bias_sum ? plan.nt : 0, tiles = plan.mt * plan.nt;
+  const size_t others = u.n > r0 ? (u.n - r0 + kUpdateBlock - 1) / kUpdateBlock : 0;
+  if (sums + tiles + others > INT32_MAX) return false;
+  std::string pname;
+  if (ctx->prof.enabled)
+    pname = kernel_name(plan, true, false, K, ctx->num_cus) + "_update " + std::to_string(K) + "x" + std::to_string(N) +
+            "x" + std::to_string(B);
+  ProfScope ps(ctx, pname.c_str(), 2.0 * (double)B * K * N,
+               4.0 * (double)(B * K + B * N) + (u.adamw ? 28.0 : 12.0) * (double)u.n);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(sums + tiles + others)), dim3(256), 0, ctx->stream, w, u, (int)sums,
+                       (int)tiles, (int)plan.nt, bias, r0);
+  };
+#define UPDATE_LAUNCH_AS(T_, UA_, ONE_)                                     \
+  do {                                                                      \
+    if (u.adamw) launch(gemm_tile_update_kernel<T_, UA_, ONE_, true>);      \
+    else launch(gemm_tile_update_kernel<T_, UA_, ONE_, false>);             \
+  } while (0)
+#define UPDATE_LAUNCH(T_)                                     \
+  do {                                                        \
+    const bool one = B <= 4096 / T_;                          \
+    if (plan.ua && one) UPDATE_LAUNCH_AS(T_, true, true);     \
+    else if (plan.ua) UPDATE_LAUNCH_AS(T_, true, false);      \
+    else if (one) UPDATE_LAUNCH_AS(T_, false, true);          \
+    else UPDATE_LAUNCH_AS(T_, false, false);                  \
+  } while (0)
+  if (plan.tile == 16) UPDATE_LAUNCH(16);
+  else if (plan.tile == 32) UPDATE_LAUNCH(32);
+  else UPDATE_LAUNCH(64);
+#undef UPDATE_LAUNCH
+#undef UPDATE_LAUNCH_AS
   ORCA_HIP_CHECK(hipGetLastError());
   return true;
 }

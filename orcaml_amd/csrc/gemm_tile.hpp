@@ -51,8 +51,19 @@ constexpr int tile_slab_floats() {
   return TileOperand<T, !TA, UA>::FLOATS + TileOperand<T, TB, UA>::FLOATS;
 }
 
-template <int T, bool TA, bool TB, bool UA, bool ONE>
-__device__ __forceinline__ void tile_product(const GemmParams& p, int bx, int by, int bz, float* __restrict__ smem) {
+struct NoUpdate {
+  static constexpr bool used = false;
+  template <int E>
+  struct State {};
+  template <int E>
+  __device__ __forceinline__ void load(State<E>&, int, size_t) const {}
+};
+
+// U: what becomes of an element of C and of a column sum besides being stored (NoUpdate, or
+// TileUpdate below; whole products without an epilogue only).
+template <int T, bool TA, bool TB, bool UA, bool ONE, class U = NoUpdate>
+__device__ __forceinline__ void tile_product(const GemmParams& p, int bx, int by, int bz, float* __restrict__ smem,
+                                             const U& upd = U()) {
   using OpA = TileOperand<T, !TA, UA>;
   using OpB = TileOperand<T, TB, UA>;
   constexpr int KS = OpA::KS;
@@ -92,7 +103,10 @@ __device__ __forceinline__ void tile_product(const GemmParams& p, int bx, int by
           }
           if (more) __syncthreads();
         });
-    if (tid < T && n0 + tid < p.N) p.colsum[n0 + tid] = cs;
+    if (tid < T && n0 + tid < p.N) {
+      p.colsum[n0 + tid] = cs;
+      if constexpr (U::used) upd.bias(n0 + tid, cs);
+    }
     return;
   }
 
@@ -114,6 +128,18 @@ __device__ __forceinline__ void tile_product(const GemmParams& p, int bx, int by
   for (int c = 0; c < 2; ++c)
 #pragma unroll
     for (int r = 0; r < (T == 16 ? 4 : 16); ++r) acc[c][r] = 0.0f;
+
+  // An updated element's state is loaded before the product where that is a few registers.
+  constexpr int NU = T == 64 ? 16 : T * T / 256;  // elements per thread
+  [[maybe_unused]] typename U::template State<NU> us;
+  [[maybe_unused]] const int u_row = T == 64 ? m0 + (wave >> 1) * 32 + g * 4 : m0 + tid / T, u_col = T == 64 ? n0 + rb : n0 + tid % T;
+  [[maybe_unused]] auto row_of = [&](int e) { return T == 64 ? u_row + (e >> 2) * 8 + (e & 3) : u_row + 256 / T * e; };
+  [[maybe_unused]] auto load_update = [&]() {
+#pragma unroll
+    for (int e = 0; e < NU; ++e)
+      upd.load(us, e, (size_t)min(row_of(e), p.M - 1) * p.ldc + min(u_col, p.N - 1));
+  };
+  if constexpr (U::used && T < 64) load_update();
 
   constexpr int HS = T == 64 ? 16 : 8;  // MFMA steps in half a slab
   float fa[2][HS], fb[2][HS];
@@ -181,6 +207,13 @@ __device__ __forceinline__ void tile_product(const GemmParams& p, int bx, int by
     floatx16 sum[1][1];
 #pragma unroll
     for (int r = 0; r < 16; ++r) sum[0][0][r] = acc[0][r] + acc[1][r];
+    if constexpr (U::used) {
+      load_update();
+#pragma unroll
+      for (int e = 0; e < NU; ++e)
+        if (row_of(e) < p.M && u_col < p.N) upd.store(us, e, (size_t)row_of(e) * p.ldc + u_col, sum[0][0][e]);
+      return;
+    }
     write_tile(sum, C, ldc, epi, m0 + (wave >> 1) * 32, n0 + (wave & 1) * 32, m0 + T <= p.M && n0 + T <= p.N, p);
   } else {
     __syncthreads();  // the last slab's fragments are read
@@ -198,7 +231,12 @@ __device__ __forceinline__ void tile_product(const GemmParams& p, int bx, int by
       const int o = tid + 256 * e;
       const int row = m0 + o / T;
       const float v = ((smem[o] + smem[o + T * T]) + smem[o + 2 * T * T]) + smem[o + 3 * T * T];
-      if (row < p.M && col < p.N) tile_store_one(p, C, ldc, epi, row, col, v);
+      if (row < p.M && col < p.N) {
+        if constexpr (U::used)
+          upd.store(us, e, (size_t)row * p.ldc + col, v);
+        else
+          tile_store_one(p, C, ldc, epi, row, col, v);
+      }
     }
   }
 }
@@ -226,5 +264,104 @@ __global__ void __launch_bounds__(256, 2) gemm_tile_pair_kernel(GemmParams x, Ge
   } else {
     const int by = b < 0 ? (w.M + TW - 1) / TW : c / w_nt;
     tile_product<TW, true, false, UA, false>(w, b < 0 ? (int)blockIdx.x : c % w_nt, by, 0, smem);
+  }
+}
+
+// A model's whole optimizer step in the launch of its last product, dW of layer 0: column sums
+// (w_sums blocks), dW's tiles (w_blocks), whose blocks update the elements that they produce,
+// and the rest of the arenas, elements [rest, u.n), 4096 a block.  Nothing else of the step
+// reads W_0, and dW reads no parameter, so the update needs no pass of its own: its memory
+// traffic runs beside the product, W_0's gradient is not read back, and the launch with its
+// start and drain goes.  Same arithmetic per element as the passes in fused.hip, same bits.
+// 64 SGD steps of 784-128-128-10 / B 64 with a read 2219 -> 2084 us, 32 AdamW steps of
+// 784-1024-1024-10 / B 256 2820 -> 2753 us and of 500-1001-333-26 / B 200 2558 -> 2441 us.
+template <bool ADAMW>
+struct TileUpdate {
+  static constexpr bool used = true;
+  template <int E>
+  struct State {
+    float p[E], m[E], v[E];
+  };
+  const ArenaUpdate& u;
+  const AdamWScalars& k;
+  size_t b0;  // the bias's first element
+
+  template <int E>
+  __device__ __forceinline__ void load(State<E>& s, int e, size_t i) const {
+    s.p[e] = u.P[i];
+    if (ADAMW) {
+      s.m[e] = u.M[i];
+      s.v[e] = u.V[i];
+    }
+  }
+  template <int E>
+  __device__ __forceinline__ void store(State<E>& s, int e, size_t i, float g) const {
+    u.G[i] = g;
+    if (ADAMW) {
+      adamw_elem(s.p[e], g, s.m[e], s.v[e], k);
+      u.M[i] = s.m[e];
+      u.V[i] = s.v[e];
+      u.P[i] = s.p[e];
+    } else {
+      u.P[i] = s.p[e] - g * k.lr;
+    }
+  }
+  __device__ __forceinline__ void bias(int c, float g) const {
+    State<1> s;
+    load(s, 0, b0 + c);
+    store(s, 0, b0 + c, g);
+  }
+};
+
+constexpr int kUpdateBlock = 4096;  // arena elements per updating block: four float4 of each array per thread
+
+template <int T, bool UA, bool ONE, bool ADAMW>
+__global__ void __launch_bounds__(256, ONE ? 4 : 2)
+    gemm_tile_update_kernel(GemmParams w, ArenaUpdate u, int w_sums, int w_blocks, int w_nt, size_t bias, size_t rest) {
+  __shared__ __attribute__((aligned(16))) float smem[(ONE ? 1 : 2) * tile_slab_floats<T, true, false, UA>()];
+  const AdamWScalars k = u.kdev ? *u.kdev : u.k;
+  const int b = (int)blockIdx.x - w_sums, c = b - w_blocks;
+  if (c < 0) {
+    const int by = b < 0 ? (w.M + T - 1) / T : b / w_nt;
+    tile_product<T, true, false, UA, ONE>(w, b < 0 ? (int)blockIdx.x : b % w_nt, by, 0, smem,
+                                          TileUpdate<ADAMW>{u, k, bias});
+    return;
+  }
+  // arena offsets are multiples of 64 elements, so every group of four is whole
+  const size_t i0 = rest + (size_t)c * kUpdateBlock + threadIdx.x * 4;
+  floatx4 p[4], g[4], m[4], v[4];
+  auto ld = [&](const float* a, int j) {
+    return __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(a + min(i0 + 1024 * j, u.n - 4)));
+  };
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    p[j] = ld(u.P, j);
+    g[j] = ld(u.G, j);
+    if (ADAMW) {
+      m[j] = ld(u.M, j);
+      v[j] = ld(u.V, j);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const size_t i = i0 + 1024 * j;
+    if (i >= u.n) return;
+    auto st = [&](float* a, floatx4 x) { __builtin_nontemporal_store(x, reinterpret_cast<floatx4*>(a + i)); };
+    if (ADAMW) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float pe = p[j][e], me = m[j][e], ve = v[j][e];
+        adamw_elem(pe, g[j][e], me, ve, k);
+        p[j][e] = pe;
+        m[j][e] = me;
+        v[j][e] = ve;
+      }
+      st(u.M, m[j]);
+      st(u.V, v[j]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p[j][e] = p[j][e] - g[j][e] * k.lr;
+    }
+    st(u.P, p[j]);
   }
 }

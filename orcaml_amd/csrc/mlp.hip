@@ -194,7 +194,7 @@ void step_body(orca_hip_mlp* m, const AdamWScalars* kdev) {
   // whether this step's update of layers >= 1 runs on the second stream
   const bool overlap = m->side && split > 0 &&
                        (m->shard_count == 1 || (m->arena - split) / m->shard_count >= kMinShardOverlapParams);
-  bool forked = false;
+  bool forked = false, updated = false;
   // With a second arena the update writes P_next and reads P.
   float* P_out = m->P_next ? m->P_next : m->P;
   auto update_range = [&](size_t begin, size_t end, hipStream_t stream, int bpc) {
@@ -244,6 +244,23 @@ void step_body(orca_hip_mlp* m, const AdamWScalars* kdev) {
       ping ^= 1;
       continue;
     }
+    // Small first layers: the whole update in the launch of layer 0's weight gradient.
+    if (l == 0 && !m->side && m->shard_count == 1) {
+      ArenaUpdate u{};
+      u.adamw = m->opt.kind == 1;
+      u.P = m->P;
+      u.G = m->G;
+      u.M = m->Mo;
+      u.V = m->Vo;
+      u.n = m->arena;
+      u.kdev = u.adamw ? kdev : nullptr;
+      if (u.adamw && !kdev)
+        u.k = adamw_scalars(m->opt.lr, m->opt.beta1, m->opt.beta2, m->opt.eps, m->opt.weight_decay, m->t);
+      else
+        u.k.lr = (float)m->opt.lr;
+      updated = gemm_first_layer_update(ctx, B, K, N, a, g, ew.colsum != nullptr, m->off[1], L > 1 ? m->off[2] : m->arena, u);
+      if (updated) break;
+    }
     // Layers >= 1 have all their gradients after dW of layer 1; with a second
     // arena nothing of this step writes the P that layer 1's dZ reads.
     const bool early = l == 1 && m->P_next && overlap;
@@ -287,7 +304,7 @@ void step_body(orca_hip_mlp* m, const AdamWScalars* kdev) {
     update(0, split, ctx->stream, m->u0_bpc);
     if (m->P_next) update(split + m->side_a + m->side_b, m->arena, ctx->stream, m->u0_bpc);
     ORCA_HIP_CHECK(hipStreamWaitEvent(ctx->stream, m->join, 0));
-  } else {
+  } else if (!updated) {
     update(0, m->arena, ctx->stream);
   }
 }

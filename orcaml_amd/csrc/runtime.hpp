@@ -399,6 +399,30 @@ void gemm(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t N, siz
 bool gemm_linear_backward(orca_hip_ctx* ctx, size_t B, size_t K, size_t N, const float* X, const float* dY,
                           const float* W, const float* mask, float* dX, float* dW, float* colsum);
 
+// AdamW's per-step f32 scalars.
+struct AdamWScalars {
+  float decay, b1, omb1, b2, omb2, c1, c2, eps, lr;
+};
+
+// An optimizer step over a model's arenas, W_0 at their start (the moments are AdamW's).
+struct ArenaUpdate {
+  bool adamw;
+  float* P;
+  float* G;
+  float* M;
+  float* V;
+  size_t n;                 // arena elements
+  AdamWScalars k;           // AdamW's scalars, unless kdev is set; lr for both kinds
+  const AdamWScalars* kdev;
+};
+
+// dW = X^T dY of a model's first layer (and, when bias_sum, the bias gradient), written to
+// u.G, and the optimizer step of the whole model in the same launch, where the product runs
+// unsplit on small tiles (false: nothing done).  W is [K][N] at the arenas' start, its bias at
+// element `bias`, the later layers from element `rest`, with their gradients in place.
+bool gemm_first_layer_update(orca_hip_ctx* ctx, size_t B, size_t K, size_t N, const float* X, const float* dY,
+                             bool bias_sum, size_t bias, size_t rest, const ArenaUpdate& u);
+
 // row_loss / row_correct: optional caller-owned [B] workspaces (else from the context cache).
 void softmax_ce(orca_hip_ctx* ctx, const float* logits, size_t B, size_t C, const float* onehot,
                 const int32_t* labels, float* loss, float* dlogits, int32_t* preds, int64_t* correct,
@@ -423,11 +447,8 @@ void head_backward(orca_hip_ctx* ctx, const float* H, size_t B, size_t K, const 
                    const float* dlogits, bool mask, float* dH, float* dW, float* db, const HeadWorkspace* finish,
                    float* loss, int64_t* correct, float* dh_colsum = nullptr);
 
-// AdamW's per-step f32 scalars: the f64 expressions of python/orca/optim/adamw.py:64-94
-// rounded to f32 as PyO3 passes them.
-struct AdamWScalars {
-  float decay, b1, omb1, b2, omb2, c1, c2, eps, lr;
-};
+// AdamW's scalars of step t: the f64 expressions of python/orca/optim/adamw.py:64-94 rounded to
+// f32 as PyO3 passes them.
 AdamWScalars adamw_scalars(double lr, double b1, double b2, double eps, double wd, int64_t t);
 // Writes s to device memory `dst` with a one-thread kernel on `stream` (by-value
 // argument: a captured graph that reads dst sees each step's values).

@@ -30,7 +30,7 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef floatx4 floatx4_u __attribute__((aligned(4)));
 
 // The four floats that start d places into v (d = 0 .. 3; the rest is don't care).
-__device__ __forceinline__ floatx4 shift_down(const floatx4& v, int d) {
+__device__ __forceinline__ floatx4 shift_down(floatx4 v, int d) {
   floatx4 x;
   x.x = d == 0 ? v.x : d == 1 ? v.y : d == 2 ? v.z : v.w;
   x.y = d == 0 ? v.y : d == 1 ? v.z : v.w;
