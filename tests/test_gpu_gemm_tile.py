@@ -146,6 +146,23 @@ def test_every_tile_batched(tctx, batch, M, N, K):
         np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("batch,m,k,n", [(3, 33, 20, 65), (5, 197, 64, 197), (7, 70, 300, 40), (2, 16, 5, 18), (9, 130, 70, 31)])
+def test_batched_tiles_in_any_number(ctx, batch, m, k, n):
+    """Tile counts that are no multiple of the eight XCDs, each operand transposed in turn."""
+    from orcaml_amd.backend import HipBackend
+
+    rng = np.random.default_rng(batch * m + n)
+    be = HipBackend(ctx)
+    A, B = int_matrix(rng, (batch, m, k), -3, 4), int_matrix(rng, (batch, k, n), -3, 4)
+    for ta, tb in ((0, 0), (1, 0), (0, 1)):
+        a = be.from_f32_slice((batch, k, m) if ta else (batch, m, k), np.ascontiguousarray(A.swapaxes(1, 2)) if ta else A)
+        b = be.from_f32_slice((batch, n, k) if tb else (batch, k, n), np.ascontiguousarray(B.swapaxes(1, 2)) if tb else B)
+        a = be.transpose(a, (batch, k, m), 1, 2) if ta else a
+        b = be.transpose(b, (batch, n, k), 1, 2) if tb else b
+        out = np.asarray(be.to_f32_vec(be.matmul(a, b, (batch, m, k), (batch, k, n)))).reshape(batch, m, n)
+        np.testing.assert_array_equal(out, A @ B)
+
+
 def test_more_rows_than_grid_rows_of_small_tiles(ctx):
     """2^21 + 3 rows: 32-row tiles, the cheapest for this width, would need 65537 grid rows."""
     rng = np.random.default_rng(5)
