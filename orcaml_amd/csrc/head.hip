@@ -16,9 +16,10 @@
 //                         1624-1646), reading H once.
 //
 // Both are deterministic: every sum runs in a fixed order.  The mean loss
-// needs every row's term, so it is added up after the forward kernel: by
-// block 0 of the backward kernel in a training step, or by a one-block
-// kernel when the forward runs alone.
+// needs every row's term, so it is added up after the forward kernel: by a
+// block of the backward kernel in a training step (one of its own where a CU
+// is free for it, else block 0), or by a one-block kernel when the forward
+// runs alone.
 #include <cstdint>
 
 #include "ce_row.hpp"
@@ -288,10 +289,11 @@ struct HeadBwdParams {
   float* dW;        // [K][C]
   float* db;        // [C] or null
   float* dh_colsum; // [K] column sums of dH (the bias gradient of the layer below) or null
-  HeadFinish fin;   // block 0 also finishes the forward's loss when fin.loss or fin.correct is set
+  HeadFinish fin;   // the forward's loss is finished here too when fin.loss or fin.correct is set
   int B, K;
   int mask;
   int dl_vec;  // dl is 16-byte aligned: staged with float4 loads
+  int panels;  // blocks of the product; with one block more that one finishes the loss, else block 0 does
 };
 
 // Block = 16 columns of H (a panel) x all B rows, so no block depends on
@@ -315,12 +317,20 @@ __global__ void __launch_bounds__(BWD_THREADS) head_backward_kernel(HeadBwdParam
   constexpr int BWD_GROUP = BWD_ROW_LANES * BWD_ROWS;
   constexpr int SPT = (BWD_GROUP * C / 4 + BWD_THREADS - 1) / BWD_THREADS;  // staged float4s per thread
   __shared__ __attribute__((aligned(16))) float dls[BWD_GROUP * C];
-  __shared__ float part[NW * 4 * NV];
+  __shared__ float part[NW * 4 * (NV + 4 + C)];  // the waves' sums of dW, of dH's columns and of db
+  float* const part_dz = part + NW * 4 * NV;
+  float* const part_db = part_dz + NW * 4 * 4;
   __shared__ float red_f[NW];
   __shared__ int red_i[NW];
   const int tid = threadIdx.x, wave = tid >> 6;
+  const bool finish = (p.fin.loss || p.fin.correct) && (int)blockIdx.x == ((int)gridDim.x > p.panels ? p.panels : 0);
+  if ((int)blockIdx.x >= p.panels) {
+    if (finish)
+      finish_rows(p.fin.row_loss, p.fin.row_correct, p.B, p.fin.inv_b, p.fin.loss, p.fin.correct, red_f, red_i);
+    return;
+  }
   const int q = tid & 3, rl = tid >> 2;
-  const int panel = xcd_local_index(blockIdx.x, gridDim.x);
+  const int panel = xcd_local_index(blockIdx.x, p.panels);
   const int k0 = panel * HEAD_PANEL;
   const int k = k0 + 4 * q;
   const bool kin = k < p.K;
@@ -441,7 +451,10 @@ __global__ void __launch_bounds__(BWD_THREADS) head_backward_kernel(HeadBwdParam
   // dW entry (4 q + e, c) = the sum over all row lanes of acc[e * C + c] on
   // the threads with that q.  Lane bits 2..5 are the wave's 16 row lanes and
   // bits 0..1 are q, so the fold runs over bits 32..4; part row (wave, q).
+  // The column sums of dH and of dlogits are folded the same way before the one barrier.
   fold_to_lds<NV, 32, 4>(acc, part, NV, wave * 4 + q);
+  if (p.dh_colsum) fold_to_lds<4, 32, 4>(adz, part_dz, 4, wave * 4 + q);
+  if (do_db) fold_to_lds<C, 32, 4>(adb, part_db, C, wave * 4 + q);
   __syncthreads();
   if (tid < 4 * NV) {  // tid = q * NV + j: dW[k0 + 4 q + j / C][j % C] = dW[k0 * C + tid]
     const int qq = tid / NV, j = tid % NV;
@@ -450,31 +463,22 @@ __global__ void __launch_bounds__(BWD_THREADS) head_backward_kernel(HeadBwdParam
     for (int w2 = 1; w2 < NW; ++w2) v = v + part[(w2 * 4 + qq) * NV + j];
     if (k0 + 4 * qq + j / C < p.K) p.dW[(int64_t)k0 * C + tid] = v;
   }
-  if (p.dh_colsum) {
-    __syncthreads();  // part is read above
-    fold_to_lds<4, 32, 4>(adz, part, 4, wave * 4 + q);
-    __syncthreads();
-    if (tid < 16) {  // column k0 + tid = k0 + 4 qq + e
-      const int qq = tid / 4, e = tid % 4;
-      float v = part[qq * 4 + e];
+  // other waves than dW's (16 C threads) add these
+  const int t2 = tid - (BWD_THREADS - 128), t3 = tid - (BWD_THREADS - 64);
+  if (p.dh_colsum && t2 >= 0 && t2 < 16) {  // column k0 + t2 = k0 + 4 qq + e
+    const int qq = t2 / 4, e = t2 % 4;
+    float v = part_dz[qq * 4 + e];
 #pragma unroll
-      for (int w2 = 1; w2 < NW; ++w2) v = v + part[(w2 * 4 + qq) * 4 + e];
-      if (k0 + tid < p.K) p.dh_colsum[k0 + tid] = v;
-    }
+    for (int w2 = 1; w2 < NW; ++w2) v = v + part_dz[(w2 * 4 + qq) * 4 + e];
+    if (k0 + t2 < p.K) p.dh_colsum[k0 + t2] = v;
   }
-  if (do_db) {
-    __syncthreads();
-    fold_to_lds<C, 32, 4>(adb, part, C, wave * 4 + q);
-    __syncthreads();
-    if (tid < C) {  // the q = 0 rows of part hold the partial sums
-      float v = part[tid];
+  if (do_db && t3 >= 0 && t3 < C) {  // the q = 0 rows of part_db hold the partial sums
+    float v = part_db[t3];
 #pragma unroll
-      for (int w2 = 1; w2 < NW; ++w2) v = v + part[w2 * 4 * C + tid];
-      p.db[tid] = v;
-    }
+    for (int w2 = 1; w2 < NW; ++w2) v = v + part_db[w2 * 4 * C + t3];
+    p.db[t3] = v;
   }
-  if (blockIdx.x == 0 && (p.fin.loss || p.fin.correct)) {
-    __syncthreads();
+  if (finish) {
     finish_rows(p.fin.row_loss, p.fin.row_correct, p.B, p.fin.inv_b, p.fin.loss, p.fin.correct, red_f, red_i);
   }
 }
@@ -556,7 +560,12 @@ void head_backward(orca_hip_ctx* ctx, const float* H, size_t B, size_t K, const 
   p.K = (int)K;
   p.mask = mask ? 1 : 0;
   p.dl_vec = aligned16(dlogits) ? 1 : 0;
-  const dim3 grid((unsigned)panels);
+  p.panels = (int)panels;
+  // One block fits a CU: with all CUs taken a block of its own would come after the others.
+  // With a CU free it takes the loss's reads and adds out of block 0, which has db as well
+  // (with the folds under one barrier: a step of 784-128-128-10 / B 64 32.5 -> 31.6 us).
+  const bool finish_block = finish && (loss || correct) && panels < (size_t)ctx->num_cus;
+  const dim3 grid((unsigned)(panels + (finish_block ? 1 : 0)));
   ProfScope ps(ctx, "head_bwd", 4.0 * (double)B * K * C,
                4.0 * ((double)B * K * (dH ? 2 : 1) + (double)B * C + 2.0 * K * C + C));
   switch (C) {
