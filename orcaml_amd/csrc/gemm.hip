@@ -2032,6 +2032,13 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
     else if (!trans_b) launch(gemm_tile_kernel<T_, true, false, UA_, ONE_>);              \
     else launch(gemm_tile_kernel<T_, true, true, UA_, ONE_>);                             \
   } while (0)
+#define TILE_BATCH_LAUNCH(UA_, ONE_)                                                 \
+  do {                                                                               \
+    if (!trans_a && !trans_b) launch(gemm_tile_batch_kernel<false, false, UA_, ONE_>); \
+    else if (!trans_a) launch(gemm_tile_batch_kernel<false, true, UA_, ONE_>);         \
+    else if (!trans_b) launch(gemm_tile_batch_kernel<true, false, UA_, ONE_>);         \
+    else launch(gemm_tile_batch_kernel<true, true, UA_, ONE_>);                        \
+  } while (0)
 #define TILE_LAUNCH(T_)                                   \
   do {                                                    \
     const bool one = K <= 4096 / T_;                      \
@@ -2072,7 +2079,12 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
       bound = bind;
       if (plan.tile == 16) TILE_LAUNCH(16);
       else if (plan.tile == 32) TILE_LAUNCH(32);
-      else TILE_LAUNCH(64);
+      else if (batch > 1) {
+        if (plan.ua && K <= 64) TILE_BATCH_LAUNCH(true, true);
+        else if (plan.ua) TILE_BATCH_LAUNCH(true, false);
+        else if (K <= 64) TILE_BATCH_LAUNCH(false, true);
+        else TILE_BATCH_LAUNCH(false, false);
+      } else TILE_LAUNCH(64);
     } else if (bn == 128) {
       GEMM_DISPATCH(128, 128);
     } else {
@@ -2082,6 +2094,7 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
 #undef FAST_LAUNCH
 #undef TILE_LAUNCH
 #undef TILE_LAUNCH_UA
+#undef TILE_BATCH_LAUNCH
 #undef GEMM_DISPATCH
 #undef GEMM_LAUNCH
     ORCA_HIP_CHECK(hipGetLastError());

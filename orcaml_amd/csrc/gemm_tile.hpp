@@ -241,28 +241,28 @@ __device__ __forceinline__ void tile_product(const GemmParams& p, int bx, int by
   }
 }
 
-// Consecutive workgroups go round the eight XCDs, each with its own L2.  This order gives an
-// XCD one run of consecutive tiles instead, so that the tiles of a batch entry, which share
-// its operands, read them through one L2: 96 x [197 x 64] x [64 x 197] and both gradients
-// 50.2 -> 46.8 us, 32 x [512 x 64] x [64 x 512] 47.2 -> 44.4.  (A single product keeps the
-// dispatch order, in which an XCD has every eighth column of tiles and all of its rows.)
-__device__ __forceinline__ uint32_t xcd_run(uint32_t l, uint32_t blocks) {
-  const uint32_t xcd = l % 8, rest = blocks % 8;
-  return xcd * (blocks / 8) + (xcd < rest ? xcd : rest) + l / 8;
-}
-
 template <int T, bool TA, bool TB, bool UA, bool ONE>
 __global__ void __launch_bounds__(256, ONE ? 4 : 2) gemm_tile_kernel(GemmParams p) {
   __shared__ __attribute__((aligned(16))) float smem[(ONE ? 1 : 2) * tile_slab_floats<T, TA, TB, UA>()];
-  if (p.sa || p.sb) {  // batched: see xcd_run
-    const uint32_t nx = gridDim.x, ny = gridDim.y, per = nx * ny;
-    const uint32_t id = xcd_run(blockIdx.x + nx * blockIdx.y + per * blockIdx.z, per * gridDim.z), in = id % per;
-    tile_product<T, TA, TB, UA, ONE>(p, in % nx, in / nx, id / per, smem);
-    return;
-  }
   // the column sums' chain of adds starts first
   const int by = TB || !p.colsum ? blockIdx.y : blockIdx.y ? blockIdx.y - 1 : (p.M + T - 1) / T;
   tile_product<T, TA, TB, UA, ONE>(p, blockIdx.x, by, blockIdx.z, smem);
+}
+
+// The same for a batched product on 64 x 64 tiles.  Consecutive workgroups go round the eight
+// XCDs, each with its own L2; here an XCD takes one run of consecutive tiles instead, so that
+// the tiles of a batch entry, which share its operands, read them through one L2: 96 x [197 x
+// 64] x [64 x 197] and both gradients 50.2 -> 46.8 us, 32 x [512 x 64] x [64 x 512] 47.2 ->
+// 44.4.  (Entries of smaller tiles: no difference.  A single product keeps the dispatch order,
+// in which an XCD has every eighth column of tiles with all of its rows, and a kernel without
+// this arithmetic: as a branch of one kernel it cost single products 0.2 us a launch.)
+template <bool TA, bool TB, bool UA, bool ONE>
+__global__ void __launch_bounds__(256, ONE ? 4 : 2) gemm_tile_batch_kernel(GemmParams p) {
+  __shared__ __attribute__((aligned(16))) float smem[(ONE ? 1 : 2) * tile_slab_floats<64, TA, TB, UA>()];
+  const uint32_t nx = gridDim.x, per = nx * gridDim.y, blocks = per * gridDim.z;
+  const uint32_t l = blockIdx.x + nx * blockIdx.y + per * blockIdx.z, xcd = l % 8;
+  const uint32_t id = xcd * (blocks / 8) + min(xcd, blocks % 8) + l / 8, in = id % per;
+  tile_product<64, TA, TB, UA, ONE>(p, in % nx, in / nx, id / per, smem);
 }
 
 // A Linear layer's two backward products from one grid: the column sums of dW = X^T dY (w;
