@@ -1437,13 +1437,14 @@ struct GemmPlan {
   double us;            // choose_tile's estimate (0: it was not asked)
 };
 
-// Profiler names: "gemm_<op(A)><op(B)>", with "_pipe" on 16-byte aligned operands, "_skinny"
-// for few-row products whose 32 x 32 tiles cover half the CUs or more; plain for 64 x 64
-// tiles, unaligned operands and the generic kernel.
-std::string kernel_name(const GemmPlan& g, bool ta, bool tb, size_t M, size_t cus) {
+// Profiler names: "gemm_<op(A)><op(B)>" and the kernel: "_pipe" (pipelined, 128 x 128 tiles) or
+// "_t16", "_t32", "_t64" (small tiles), with "_ua" on operands that are not 16-byte aligned;
+// nothing more for the generic kernel.
+std::string kernel_name(const GemmPlan& g, bool ta, bool tb) {
   std::string name = std::string("gemm_") + (ta ? "t" : "n") + (tb ? "t" : "n");
-  if (g.tile == 32 && !ta && M <= 256 && 2 * g.mt * g.nt >= cus) return name + "_skinny";
-  return (g.fast || g.tile) && !g.ua && g.tile != 64 ? name + "_pipe" : name;
+  if (g.tile) name += "_t" + std::to_string(g.tile);
+  else if (g.fast) name += "_pipe";
+  return g.ua && (g.tile || g.fast) ? name + "_ua" : name;
 }
 
 // The tile and K split of a product on the pipelined or small-tile kernels: the candidate
@@ -1826,7 +1827,8 @@ bool gemm_linear_backward(orca_hip_ctx* ctx, size_t B, size_t K, size_t N, const
   if (x_blocks + w_blocks > INT32_MAX) return false;
   std::string pname;
   if (ctx->prof.enabled)
-    pname = "gemm_linear_bw " + std::to_string(B) + "x" + std::to_string(K) + "x" + std::to_string(N);
+    pname = "gemm_linear_bw_t" + std::to_string(tx) + "_t" + std::to_string(tw) + (ua ? "_ua " : " ") + std::to_string(B) + "x" +
+            std::to_string(K) + "x" + std::to_string(N);
   ProfScope ps(ctx, pname.c_str(), 4.0 * (double)B * K * N, 4.0 * (double)(2 * B * N + 2 * K * N + 3 * B * K));
 #define PAIR_LAUNCH(TX_, TW_)                                                                                        \
   do {                                                                                                               \
@@ -1870,7 +1872,7 @@ bool gemm_first_layer_update(orca_hip_ctx* ctx, size_t B, size_t K, size_t N, co
   if (sums + tiles + others > INT32_MAX) return false;
   std::string pname;
   if (ctx->prof.enabled)
-    pname = kernel_name(plan, true, false, K, ctx->num_cus) + "_update " + std::to_string(K) + "x" + std::to_string(N) +
+    pname = kernel_name(plan, true, false) + "_update " + std::to_string(K) + "x" + std::to_string(N) +
             "x" + std::to_string(B);
   ProfScope ps(ctx, pname.c_str(), 2.0 * (double)B * K * N,
                4.0 * (double)(B * K + B * N) + (u.adamw ? 28.0 : 12.0) * (double)u.n);
@@ -1995,7 +1997,7 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
     if (ctx->prof.enabled) {
       pname = std::string(plan.band == 1 + BAND_EIGHT     ? "gemm_tn_band8"
                           : plan.band == 1 + BAND_ROWS112 ? "gemm_tn_band112"
-                                                          : kernel_name(plan, trans_a, trans_b, M, ctx->num_cus)) +
+                                                          : kernel_name(plan, trans_a, trans_b)) +
               " " +
               std::to_string(M) + "x" + std::to_string(N) + "x" + std::to_string(K);
       if (batch > 1) pname += "x" + std::to_string(batch);

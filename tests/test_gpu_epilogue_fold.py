@@ -34,11 +34,11 @@ def gemm_pre(ctx, A_, B_, bias):
 @pytest.mark.parametrize("M,N,K", [
     (256, 384, 160),    # pipelined 128 x 128 kernel
     (260, 196, 164),    # pipelined, edge tiles
-    (256, 1024, 784),   # skinny kernel
+    (256, 1024, 784),   # 32 x 32 tiles
     (1024, 1024, 256),  # 64 x 64 tiles
     (128, 256, 3076),   # split K: the epilogue runs in the float4 reduce
     (130, 70, 33),      # generic kernel, unaligned
-    (129, 1029, 1021),  # skinny, ragged
+    (129, 1029, 1021),  # 32 x 32 tiles, ragged
     (64, 13, 2050),     # N <= 16 stays on the tiles (split K, scalar reduce)
 ])
 def test_bias_relu_pre_epilogue_matches_composed_ops(ctx, M, N, K):
@@ -61,7 +61,7 @@ def test_bias_relu_pre_epilogue_matches_composed_ops(ctx, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [
     (256, 384, 160),    # pipelined 128 x 128 kernel (B^T)
-    (256, 1024, 1024),  # skinny kernel (B^T)
+    (256, 1024, 1024),  # 32 x 32 tiles (B^T)
     (128, 256, 3076),   # split K: the float4 reduce
     (130, 70, 33),      # generic kernel, unaligned: the scalar reduce or the tile store
     (1024, 4096, 10),   # narrow K against B^T
@@ -198,7 +198,7 @@ def test_relu_backward_on_a_held_product(ctx):
                                    (1024, 10, 4096), (1024, 4096, 10), (64, 13, 2050)])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False)])
 def test_products_never_hold_negative_zero(ctx, M, N, K, ta, tb):
-    """Every GEMM path (pipelined, skinny, split K, generic, narrow) returns +0 where all
+    """Every GEMM path (pipelined, small tiles, split K, generic, narrow) returns +0 where all
     products are -0 (negative x +0), where a row is all -0, and where terms cancel: the
     property that lets a masked product share its buffer with its identity sum (0 + x)."""
     rng = np.random.default_rng(M + N + K + 2 * ta + tb)

@@ -78,14 +78,17 @@ def test_gemm_exact_on_integers(ctx, ta, tb, M, N, K):
 
 @pytest.mark.parametrize("ta,tb,colsum", [(False, False, False), (False, False, True), (False, True, False),
                                           (True, False, True), (True, False, False), (True, True, False)])
-def test_gemm_aligned_shapes_take_pipelined_kernel(ctx, ta, tb, colsum):
-    """Products whose M, N, K are multiples of 4 run on the pipelined 128 x 128
-    kernel (profiler name *_pipe), the rest on the generic kernel; both exact
-    on integers."""
+def test_gemm_kernel_follows_size_and_alignment(ctx, ta, tb, colsum):
+    """Products that give every CU a 128 x 128 tile run on the pipelined kernel (profiler name
+    *_pipe), smaller ones on small tiles (*_t16); *_ua when a dimension is no multiple of 4.
+    All exact on integers."""
+    if ctx.prof_report()["num_cus"] != 256:
+        pytest.skip("tile counts chosen for 256 compute units")
     rng = np.random.default_rng(3)
     name = "gemm_" + ("t" if ta else "n") + ("t" if tb else "n")
-    for (M, N, K), pipe in (((256, 384, 160), True), ((260, 196, 164), True), ((256, 384, 161), False),
-                            ((256, 202, 160), False)):
+    for (M, N, K), kernel in (((256, 384, 160), "_t16"), ((260, 196, 164), "_t16"), ((256, 384, 161), "_t16_ua"),
+                              ((256, 202, 160), "_t16_ua"), ((2048, 2048, 160), "_pipe"), ((2044, 2040, 164), "_pipe"),
+                              ((2048, 2048, 161), "_pipe_ua"), ((2046, 2042, 160), "_pipe_ua")):
         A = int_matrix(rng, (M, K))
         B = int_matrix(rng, (K, N))
         ctx.prof_reset()
@@ -94,25 +97,23 @@ def test_gemm_aligned_shapes_take_pipelined_kernel(ctx, ta, tb, colsum):
                        colsum=colsum and not tb)
         ctx.prof_enable(False)
         names = {k["name"] for k in ctx.prof_report()["kernels"]}
-        want = f"{name}_pipe {M}x{N}x{K}" if pipe else f"{name} {M}x{N}x{K}"
-        assert want in names, names
+        assert f"{name}{kernel} {M}x{N}x{K}" in names, names
         C, cs = out if colsum else (out, None)
-        np.testing.assert_array_equal(C, (A.astype(np.int64) @ B.astype(np.int64)).astype(np.float32))
+        np.testing.assert_array_equal(C, (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32))
         if cs is not None:
             np.testing.assert_array_equal(cs, O.sum_to_shape(B, (1, N)).reshape(N))
 
 
-SKINNY_SHAPES = [(256, 1024, 784), (256, 1024, 1024), (200, 1000, 1000), (256, 1024, 30), (130, 1030, 777),
+FEW_ROW_SHAPES = [(256, 1024, 784), (256, 1024, 1024), (200, 1000, 1000), (256, 1024, 30), (130, 1030, 777),
                  (129, 1029, 1021)]
 
 
 @pytest.mark.parametrize("tb", [False, True])
-@pytest.mark.parametrize("M,N,K", SKINNY_SHAPES)
-def test_gemm_skinny_exact_on_integers(ctx, tb, M, N, K):
-    """Few-row, short-K products with row-major A (the 784-1024-1024-10 / B = 256 forward and
-    dX products; ragged M, N, K; K shorter than a wave's 8-k group) run whole on the skinny
-    32 x 32 kernel (no K split, no reduce launch); exact on integers, with the column sum of
-    a row-major B taken by its own pass."""
+@pytest.mark.parametrize("M,N,K", FEW_ROW_SHAPES)
+def test_gemm_few_rows_exact_on_integers(ctx, tb, M, N, K):
+    """Few-row products with row-major A (the 784-1024-1024-10 / B = 256 forward and dX products;
+    ragged M, N, K; K shorter than a slab) run whole on 32 x 32 tiles (no K split, no reduce
+    launch); exact on integers, with the column sum of a row-major B beside them."""
     cus = ctx.prof_report()["num_cus"]
     if cus != 256:
         pytest.skip("tile counts chosen for 256 compute units")
@@ -124,7 +125,8 @@ def test_gemm_skinny_exact_on_integers(ctx, tb, M, N, K):
     out = run_gemm(ctx, False, tb, A, np.ascontiguousarray(B.T) if tb else B, colsum=not tb)
     ctx.prof_enable(False)
     names = {k["name"] for k in ctx.prof_report()["kernels"]}
-    assert ("gemm_nt_skinny" if tb else "gemm_nn_skinny") + f" {M}x{N}x{K}" in names, names
+    ua = "_ua" if M % 4 or N % 4 or K % 4 else ""
+    assert f"gemm_n{'t' if tb else 'n'}_t32{ua} {M}x{N}x{K}" in names, names
     assert "gemm_splitk_reduce" not in names
     C, cs = out if not tb else (out, None)
     np.testing.assert_array_equal(C, (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32))
@@ -133,8 +135,8 @@ def test_gemm_skinny_exact_on_integers(ctx, tb, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(256, 1024, 1024), (130, 1030, 777)])
-def test_gemm_skinny_epilogues_match_composed_ops(ctx, M, N, K):
-    """The skinny kernel's bias, bias + ReLU and ReLU-mask epilogues equal the composed ops
+def test_gemm_few_rows_epilogues_match_composed_ops(ctx, M, N, K):
+    """The 32 x 32 tiles' bias, bias + ReLU and ReLU-mask epilogues equal the composed ops
     applied to its own product, bit for bit; the product is within the f32 dot-product bound."""
     rng = np.random.default_rng(M + K)
     A = rng.standard_normal((M, K)).astype(np.float32)
@@ -157,11 +159,10 @@ def test_gemm_skinny_epilogues_match_composed_ops(ctx, M, N, K):
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("M,N,K", [(1024, 1024, 256), (784, 1024, 256), (1000, 1030, 250), (1024, 1024, 33)])
 def test_gemm_small_tiles_exact_on_integers(ctx, ta, tb, M, N, K):
-    """Short products (K <= 512) whose 128 x 128 grid leaves half the CUs idle but whose
-    64 x 64 grid covers three quarters of them run unsplit on 64 x 64 tiles (profiler name
-    without _pipe, no reduce launch): the 784-1024-1024-10 / B = 256 weight gradients,
-    ragged edges and a K that is not a multiple of the slab.  Exact on integers, with the
-    folded column sum."""
+    """Short products whose 128 x 128 grid leaves half the CUs idle run unsplit on smaller tiles
+    (no reduce launch): 64 x 64 where those cover the CUs about once (the 784-1024-1024-10 /
+    B = 256 weight gradients, ragged edges and a K that is not a multiple of the slab), 32 x 32
+    for one odd NT product.  Exact on integers, with the column sum."""
     cus = ctx.prof_report()["num_cus"]
     if cus != 256:
         pytest.skip("tile counts chosen for 256 compute units")
@@ -174,8 +175,10 @@ def test_gemm_small_tiles_exact_on_integers(ctx, ta, tb, M, N, K):
                    colsum=not tb)
     ctx.prof_enable(False)
     names = {k["name"] for k in ctx.prof_report()["kernels"]}
-    name = "gemm_" + ("t" if ta else "n") + ("t" if tb else "n") + f" {M}x{N}x{K}"
-    assert name in names and "gemm_splitk_reduce" not in names, names
+    ua = "_ua" if M % 4 or N % 4 or K % 4 else ""
+    tile = 32 if (ta, tb, M) == (False, True, 1000) else 64
+    assert f"gemm_{'t' if ta else 'n'}{'t' if tb else 'n'}_t{tile}{ua} {M}x{N}x{K}" in names, names
+    assert "gemm_splitk_reduce" not in names
     C, cs = out if not tb else (out, None)
     np.testing.assert_array_equal(C, (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32))
     if cs is not None:
@@ -208,7 +211,7 @@ def test_gemm_grid_of_half_the_cus_splits_k(ctx):
     """A 128 x 128 tile grid that covers exactly half the CUs runs as two K chunks (every CU busy,
     then the in-order chunk sum); the product stays exact on integers."""
     cus = ctx.prof_report()["num_cus"]
-    M, N, K = 128, 128 * (cus // 2), 2048  # K > 1024: neither 64 x 64 tiles nor the skinny kernel
+    M, N, K = 128, 128 * (cus // 2), 2048  # too long a K for small tiles
     rng = np.random.default_rng(11)
     A = int_matrix(rng, (M, K))
     B = int_matrix(rng, (K, N))

@@ -155,7 +155,7 @@ def test_mlp784_4096_b1024_one_adamw_step(ctx, batch):
     """784-4096-4096-10, batch 1024, one AdamW step against the oracle, end to end
     (and the 512 / 256 / 128-row shares of 2-, 4- and 8-way data parallelism: F2 and dX2
     split K in two, four and eight chunks and sum them in their reduce pass, which also
-    applies the epilogue; at 128 rows F1 runs whole on the skinny kernel; dW1 stays on the
+    applies the epilogue; at 128 rows F1 runs whole on the small tiles; dW1 stays on the
     banded kernel with K = 512, 256, 128):
     loss and logits to the path's tolerance (1e-5 abs + 1e-4 rel); gradients and
     updated parameters to that tolerance except for a reported fraction <= 1e-5
