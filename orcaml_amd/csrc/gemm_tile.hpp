@@ -195,7 +195,9 @@ __device__ __forceinline__ void tile_product(const GemmParams& p, int bx, int by
           __syncthreads();
           frags(smem + (P ^ 1) * SLAB, 0, fa[0], fb[0]);
         }
-        mfma(fa[1], fb[1]);
+        // a K up to 32 is in the first half of a one-slab 64-tile; the other would multiply zeros,
+        // 0.43 us of each wave (X^T dY of 2183 x 832 x 8: 6.3 -> 5.4 us, 2048 x 2048 x 32: 9.6 -> 7.9)
+        if (!(ONE && T == 64) || p.K > 32) mfma(fa[1], fb[1]);
         if constexpr (decltype(full)::value) interleave(std::false_type{});
       });
 

@@ -84,7 +84,8 @@ def product(ctx, ta, tb, A, B, pad=0, shift=0, colsum=False, kind=_lib.EPI_NONE,
 # M, N, K: one element past, at and short of each tile; K from less than a slab to several, whole
 # and ragged; the fewest floats the kernels take.
 SHAPES = [(17, 17, 17), (16, 32, 64), (15, 33, 255), (31, 65, 257), (64, 128, 784), (63, 129, 513), (129, 127, 300),
-          (132, 260, 36), (1, 18, 4), (4, 20, 1000), (20, 4, 131), (200, 26, 333), (130, 70, 1030)]
+          (132, 260, 36), (1, 18, 4), (4, 20, 1000), (20, 4, 131), (200, 26, 333), (130, 70, 1030),
+          (70, 130, 31), (129, 65, 32), (66, 131, 33)]  # around half of a one-slab 64-tile
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
