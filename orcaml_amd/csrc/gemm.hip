@@ -1455,12 +1455,19 @@ std::string kernel_name(const GemmPlan& g, bool ta, bool tb) {
 // The tile and K split of a product on the pipelined or small-tile kernels: the candidate
 // with the least estimated time.  A CU that gets r blocks takes
 //   3 us + r (per block + slabs per block * per slab)
-// and a split adds its reduce launch, 2.4 us and the partial sums at 5 TB/s.  X^T dY is priced
-// with its bias gradient (the plan must not depend on whether that is asked for, so that the
-// product's bits do not): a chain of adds of about 10 ns a row beside the small tiles, 0.19 us
-// a slab folded into the 128 tiles, a launch of its own after a split of those.  The
-// constants are fits to HIP-event times of back-to-back launches on 256 CUs, 66 shapes from
-// 8 x 603 x 240 to 2048^3 in all layouts, each tile and split forced in turn.  A slab is 16 KiB
+// and a split adds its reduce launch, 3 us and the partial sums at 5 TB/s.  Blocks of one slab
+// run four to a CU and hide most of each other's loads and stores, so their rounds up to the
+// fourth cost `beside` of the first and the others `after`; a 64-tile whose K ends in the slab's first half multiplies half
+// (X W of 2290 x 1128 x 10: 9.9 us on tiles of 128, 7.0 on tiles of 64).  X^T dY is priced with
+// its bias gradient (the plan must not depend on whether that is asked for, so that the
+// product's bits do not): a chain of adds beside the small tiles' product, 5 ns a row beside
+// tiles of 16 and 6.6 beside the others, 0.19 us a slab folded into the 128 tiles, a launch of
+// its own after a split of those.  Where the chain is the time, the product itself decides
+// (2560 x 48 x 2942: 31.3 us on the first candidate, 20.3 on the product's cheapest).  The
+// constants are fits to HIP-event times of back-to-back launches on 256 CUs, every candidate
+// of 2096 products from 8 to 4096 a side in the layouts of a Linear layer (a sixth of them:
+// profiles/gemm_tile_candidates.csv); the rule's choices take 1.6 % more than the best candidates
+// in the geometric mean (2.7 % without the one-slab terms and with one chain of 10.5 ns).  A slab is 16 KiB
 // of each operand; small tiles pay for row-major ("mn-fast") operands, whose rows of 16 or 32
 // floats take a memory line each, and more when those rows are not 16-byte aligned.  What the
 // small tiles lose per multiply they win by covering the CUs: 64 x 128 x 784 takes 5.3 us on
@@ -1473,20 +1480,22 @@ struct TileForm {
   int tile;
   size_t slab_k;
   double block_us;
-  double slab_us[2][3];  // [unaligned operands][row-major operands: NT; NN, TT; TN]
+  double one_slab_us, beside, after;  // one-slab blocks: what the first round saves, further rounds' shares
+  double colsum_ns;                   // a row of the column sums' chain (small tiles)
+  double slab_us[2][3];               // [unaligned operands][row-major operands: NT; NN, TT; TN]
 };
-constexpr TileForm kTileForms[4] = {{16, 256, 0.4, {{0.50, 0.60, 0.95}, {0.55, 0.70, 1.05}}},
-                                    {32, 128, 0.5, {{0.64, 0.68, 0.85}, {0.68, 0.90, 0.95}}},
-                                    {64, 64, 1.0, {{1.06, 1.06, 1.06}, {1.06, 1.10, 1.15}}},
-                                    {128, BK, 3.0, {{1.82, 1.82, 1.82}, {1.84, 1.84, 1.84}}}};
+constexpr TileForm kTileForms[4] = {{16, 256, 0.4, 0.5, 0.3, 0.7, 5.0, {{0.50, 0.60, 0.95}, {0.55, 0.70, 1.05}}},
+                                    {32, 128, 0.5, 0.3, 0.55, 0.7, 6.6, {{0.64, 0.68, 0.85}, {0.68, 0.90, 0.95}}},
+                                    {64, 64, 1.0, 0.15, 0.5, 0.5, 6.6, {{1.06, 1.06, 1.13}, {1.06, 1.10, 1.25}}},
+                                    {128, BK, 3.0, 0.0, 1.0, 1.0, 0.0, {{1.82, 1.82, 1.82}, {1.84, 1.84, 1.84}}}};
 // The chain of adds of a column sum beside small tiles, us for k rows.
-constexpr double colsum_chain_us(size_t k) { return 4.0 + 0.0105 * (double)k; }
+constexpr double colsum_chain_us(const TileForm& f, size_t k) { return 3.0 + 1e-3 * f.colsum_ns * (double)k; }
 
 void choose_tile(orca_hip_ctx* ctx, GemmPlan& g, bool trans_a, bool trans_b, size_t M, size_t N, size_t K,
                  size_t batch) {
   const size_t target = (size_t)ctx->num_cus;
   const int mn_fast = (trans_a ? 1 : 0) + (trans_b ? 0 : 1);
-  double best = 1e300;
+  double best = 1e300, best_product = 1e300;
   size_t best_chunk = K;
   for (const TileForm& f : kTileForms) {
     if (ctx->gemm_tile_bn && ctx->gemm_tile_bn != f.tile) continue;
@@ -1500,15 +1509,24 @@ void choose_tile(orca_hip_ctx* ctx, GemmPlan& g, bool trans_a, bool trans_b, siz
       const size_t per = (slabs + s - 1) / s;
       s = (slabs + per - 1) / per;
       const double rounds = (double)((tiles * s + target - 1) / target);
-      // one-slab products run four blocks a CU, which hide more of each other's loads and stores
-      double us = 3.0 + rounds * (f.block_us - (slabs == 1 && f.tile < 128 ? 0.15 : 0.0) + (double)per * f.slab_us[g.ua ? 1 : 0][mn_fast]);
-      if (s > 1) us += 2.4 + (double)(s + 1) * (double)(batch * M * N) * 4.0 / 5e6;
+      const double slab = f.slab_us[g.ua ? 1 : 0][mn_fast] * (f.tile == 64 && K <= 32 ? 0.5 : 1.0);
+      const double block = f.block_us + (double)per * slab;
+      double product = 3.0;
+      if (slabs == 1 && f.tile < 128)
+        product += block * (1.0 + f.beside * (std::min(rounds, 4.0) - 1.0) + f.after * std::max(rounds - 4.0, 0.0)) - f.one_slab_us;
+      else
+        product += block * rounds;
+      double us = product;
       if (mn_fast == 2 && batch == 1) {
-        if (f.tile < 128) us = std::max(us, colsum_chain_us(K));
+        if (f.tile < 128) us = std::max(us, colsum_chain_us(f, K));
         else us += s > 1 ? 4.0 + 0.009 * (double)K : 0.19 * (double)slabs;
       }
-      if (us < best) {
+      const double reduce = s > 1 ? 3.0 + (double)(s + 1) * (double)(batch * M * N) * 4.0 / 5e6 : 0.0;
+      us += reduce;
+      product += reduce;
+      if (us < best || (us == best && product < best_product)) {
         best = us;
+        best_product = product;
         g.tile = f.tile == 128 ? 0 : f.tile;
         g.splits = (int)s;
         best_chunk = per * f.slab_k;
@@ -1796,7 +1814,7 @@ bool gemm_linear_backward(orca_hip_ctx* ctx, size_t B, size_t K, size_t N, const
     const double bx = block(fx, 0, N), bw = block(fw, 2, B);
     const double nx = (double)tiles(B, K, (size_t)fx.tile), nw = (double)tiles(K, N, (size_t)fw.tile);
     const double longest = std::max(bx, bw), spread = (nx * bx + nw * bw) / cus + 0.5 * longest;
-    const double us = std::max(3.0 + (nx + nw <= cus ? longest : std::max(longest, spread)), colsum ? colsum_chain_us(B) : 0.0);
+    const double us = std::max(3.0 + (nx + nw <= cus ? longest : std::max(longest, spread)), colsum ? colsum_chain_us(fw, B) : 0.0);
     if (us < best_us) {
       best_us = us;
       best = i;

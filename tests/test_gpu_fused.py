@@ -160,9 +160,9 @@ def test_gemm_few_rows_epilogues_match_composed_ops(ctx, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(1024, 1024, 256), (784, 1024, 256), (1000, 1030, 250), (1024, 1024, 33)])
 def test_gemm_small_tiles_exact_on_integers(ctx, ta, tb, M, N, K):
     """Short products whose 128 x 128 grid leaves half the CUs idle run unsplit on smaller tiles
-    (no reduce launch): 64 x 64 where those cover the CUs about once (the 784-1024-1024-10 /
-    B = 256 weight gradients, ragged edges and a K that is not a multiple of the slab), 32 x 32
-    for one odd NT product.  Exact on integers, with the column sum."""
+    (no reduce launch): the 784-1024-1024-10 / B = 256 weight gradients, whose 64 x 64 tiles cover
+    the CUs about once, ragged edges and a K that is not a multiple of the slab.  Exact on
+    integers, with the column sum."""
     cus = ctx.prof_report()["num_cus"]
     if cus != 256:
         pytest.skip("tile counts chosen for 256 compute units")
@@ -176,8 +176,8 @@ def test_gemm_small_tiles_exact_on_integers(ctx, ta, tb, M, N, K):
     ctx.prof_enable(False)
     names = {k["name"] for k in ctx.prof_report()["kernels"]}
     ua = "_ua" if M % 4 or N % 4 or K % 4 else ""
-    tile = 32 if (ta, tb, M) == (False, True, 1000) else 64
-    assert f"gemm_{'t' if ta else 'n'}{'t' if tb else 'n'}_t{tile}{ua} {M}x{N}x{K}" in names, names
+    kernel, shape = f"gemm_{'t' if ta else 'n'}{'t' if tb else 'n'}", f"{ua} {M}x{N}x{K}"
+    assert names & {f"{kernel}_t{t}{shape}" for t in ((16, 32, 64) if M == 1000 else (64,))}, names
     assert "gemm_splitk_reduce" not in names
     C, cs = out if not tb else (out, None)
     np.testing.assert_array_equal(C, (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32))

@@ -164,6 +164,28 @@ def test_batched_tiles_in_any_number(ctx, batch, m, k, n):
         np.testing.assert_array_equal(out, A @ B)
 
 
+@pytest.mark.parametrize("ta,M,N,K,tiles", [
+    # the column sum's chain of adds is longer than any product: the product still takes its own cheapest tile
+    (True, 2560, 48, 2942, (32, 64)), (True, 105, 920, 3316, (32, 64)), (True, 96, 1160, 2968, (32, 64)),
+    # one round of 128-tiles against four and more one-slab 64-tiles a CU
+    (False, 2290, 1128, 10, (64,)), (False, 1064, 1960, 17, (64,)), (False, 3648, 1000, 16, (64,))])
+def test_tile_of_lopsided_products(ctx, ta, M, N, K, tiles):
+    if ctx.prof_report()["num_cus"] != 256:
+        pytest.skip("tile counts chosen for 256 compute units")
+    rng = np.random.default_rng(M + N)
+    A, B = int_matrix(rng, (M, K), -3, 4), int_matrix(rng, (K, N), -3, 4)
+    ctx.prof_reset()
+    ctx.prof_enable(True)
+    got = product(ctx, ta, False, A, B, kind=_lib.EPI_NONE if ta else _lib.EPI_RELU_MASK,
+                  mask=None if ta else np.ones((M, N), np.float32))[0]
+    ctx.prof_enable(False)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    np.testing.assert_array_equal(got, want.astype(np.float32))
+    names = {k["name"].split()[0] for k in ctx.prof_report()["kernels"]}
+    kernel = "gemm_tn" if ta else "gemm_nn"
+    assert any(n in (f"{kernel}_t{t}", f"{kernel}_t{t}_ua") for n in names for t in tiles), names
+
+
 def test_more_rows_than_grid_rows_of_small_tiles(ctx):
     """2^21 + 3 rows: 32-row tiles, the cheapest for this width, would need 65537 grid rows."""
     rng = np.random.default_rng(5)
