@@ -342,8 +342,15 @@ __global__ void __launch_bounds__(CR_THREADS)
 // is cut in four: lane r + 16 q takes columns 64 q .. 64 q + 63 of each slab, and the four are
 // combined in column order -- a strictly greater value replaces the running one, so the first
 // of equal values (of -0 and +0) is kept as in one chain.  [1024, 1000], device time: sum 40 ->
-// 6 us, maximum 41 -> 5.7 us.
+// 6 us, maximum 41 -> 5.7 us.  A block loads and combines a whole slab, most of it past the end
+// of a short row, while the lines of short rows stay in L1 from one of a thread's loads to the
+// next: [2^20, 16] takes 81 us here (maximum 98) and 45 with a thread per row.  Sums are even
+// at 24 columns ([2^16, 24] 5.7 us both, [2^18, 23] 20.0 and 21.0), maxima of 2^17 rows and more
+// too ([2^18, 24] 24.2 and 24.4 us), of fewer rows at 30 ([2^16, 28] 7.1 and 6.2 us, [2^16, 30]
+// 7.3 and 7.4).
 constexpr int RR_ROWS = 16;
+// Columns from which rows come here.
+constexpr int64_t rr_min_cols(bool is_max, size_t rows) { return is_max && rows < (size_t(1) << 17) ? 30 : 24; }
 
 template <bool IS_MAX, bool UA>
 __global__ void __launch_bounds__(256) rowreduce_kernel(const float* __restrict__ in, float* __restrict__ out, int rows,
@@ -802,9 +809,9 @@ static int reduce_entry(orca_hip_ctx* ctx, bool is_max, const void* s, const siz
         size_t n_threads = n_in / (size_t)a.red_count;
         ProfScope ps(ctx, op, 0.0, 4.0 * (n_in + n_out));
         unsigned g = (unsigned)((n_threads + 63) / 64);
-        // Contiguous rows of at least 16 values (a slab's 32-bit offsets hold 4 GiB); shorter
-        // rows are a few loads per thread.
-        const bool rows_contiguous = a.n_red == 1 && a.red_strides[0] == 1 && a.red_count >= 16 &&
+        // Contiguous rows of enough values (a slab's 32-bit offsets hold 4 GiB).
+        const bool rows_contiguous = a.n_red == 1 && a.red_strides[0] == 1 &&
+                                     a.red_count >= rr_min_cols(is_max, n_threads) &&
                                      (a.n_kept == 0 || (a.n_kept == 1 && a.kept_strides[0] == a.red_count)) &&
                                      n_in * sizeof(float) < 0xffffffffull;
         if (rows_contiguous) {
