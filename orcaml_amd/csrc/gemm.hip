@@ -1498,7 +1498,7 @@ void choose_tile(orca_hip_ctx* ctx, GemmPlan& g, bool trans_a, bool trans_b, siz
   double best = 1e300, best_product = 1e300;
   size_t best_chunk = K;
   for (const TileForm& f : kTileForms) {
-    if (ctx->gemm_tile_bn && ctx->gemm_tile_bn != f.tile) continue;
+    if (ctx->gemm_tile && ctx->gemm_tile != f.tile) continue;
     const size_t t = (size_t)f.tile;
     if (f.tile < 128 && (M + t - 1) / t >= 65535) continue;  // grid rows (and one for column sums): 2^20 rows of 16
     const size_t tiles = ((M + t - 1) / t) * ((N + t - 1) / t) * batch, slabs = (K + f.slab_k - 1) / f.slab_k;
@@ -1583,8 +1583,9 @@ GemmPlan plan_gemm(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size
   const size_t t128 = ((M + 127) / 128) * ((N + 127) / 128) * batch;
   size_t BM = 128;
   // Generic kernel tile: 128 x 128 when that gives every CU a block, else
-  // 128 x 64 (twice the blocks).
+  // 128 x 64 (twice the blocks), unless the context fixes it.
   int bn = mfma || t128 >= target ? 128 : 64;
+  if (!mfma && ctx->gemm_generic_bn) bn = ctx->gemm_generic_bn;
   // A weight gradient X^T dY (no epilogue) whose banded grid is one round between
   // half and all of the CUs (so it takes no K split) runs banded: 112-row tiles for
   // M = 112 R (R <= 7: as many tiles as 128 rows need, each 12.5 % smaller), or
@@ -1793,7 +1794,7 @@ bool narrow_linear_backward(orca_hip_ctx* ctx, const float* H, size_t B, size_t 
 // launched) when the two run apart.
 bool gemm_linear_backward(orca_hip_ctx* ctx, size_t B, size_t K, size_t N, const float* X, const float* dY,
                           const float* W, const float* mask, float* dX, float* dW, float* colsum) {
-  if (!B || !K || !N || B > INT32_MAX || K > INT32_MAX || N > INT32_MAX || ctx->gemm_tile_bn || ctx->gemm_splits) return false;
+  if (!B || !K || !N || B > INT32_MAX || K > INT32_MAX || N > INT32_MAX || ctx->gemm_tile || ctx->gemm_splits) return false;
   const GemmPlan px = plan_gemm(ctx, false, true, B, K, N, dY, N, 0, W, N, 0, 1, ORCA_HIP_EPI_RELU_MASK);
   const GemmPlan pw = plan_gemm(ctx, true, false, K, N, B, X, K, 0, dY, N, 0, 1);
   if (px.us == 0.0 || pw.us == 0.0) return false;  // narrow, banded or generic

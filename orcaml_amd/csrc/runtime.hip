@@ -125,9 +125,12 @@ int orca_hip_ctx_create(int device, orca_hip_ctx** out) {
     if (const char* v = std::getenv("ORCA_HIP_GEMM_NARROW")) ctx->gemm_narrow = v[0] != '0';
     if (const char* v = std::getenv("ORCA_HIP_GEMM_BAND")) ctx->gemm_band = v[0] == '0' ? 0 : v[0] == '1' ? 1 : 2;
     if (const char* v = std::getenv("ORCA_HIP_EW_JIT")) ctx->ew_jit_mode = v[0] == '0' ? 0 : v[0] == '2' ? 2 : 1;
+    if (const char* v = std::getenv("ORCA_HIP_GEMM_SMALL_TILES")) ctx->gemm_tile = v[0] == '0' ? 128 : 0;
     if (const char* v = std::getenv("ORCA_HIP_GEMM_TILE")) {
-      const int t = std::atoi(v);
-      if (t == 16 || t == 32 || t == 64 || t == 128) ctx->gemm_tile_bn = t;
+      for (int t : {16, 32, 64, 128})
+        if (std::to_string(t) == v) ctx->gemm_tile = t;
+      if (std::strcmp(v, "128x128") == 0) ctx->gemm_generic_bn = 128;
+      if (std::strcmp(v, "128x64") == 0) ctx->gemm_generic_bn = 64;
     }
     if (const char* v = std::getenv("ORCA_HIP_GEMM_SPLITS")) ctx->gemm_splits = std::max(0, std::min(64, std::atoi(v)));
     hipError_t e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);

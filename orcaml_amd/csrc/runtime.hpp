@@ -215,10 +215,13 @@ struct orca_hip_ctx {
   std::mutex mu;
   // Tuning switches read once when the context is created (environment):
   // ORCA_HIP_GEMM_FAST=0 sends every product through the generic GEMM kernel,
-  // ORCA_HIP_GEMM_TILE=16|32|64|128 fixes the tile of the other products (0 = by the
-  // product's size) and ORCA_HIP_GEMM_SPLITS=n their K split.
+  // ORCA_HIP_GEMM_TILE=128x128|128x64 fixes that kernel's tile (0 = by grid size),
+  // ORCA_HIP_GEMM_TILE=16|32|64|128 the tile of the other products (0 = by the product's
+  // size; any other value changes nothing) and ORCA_HIP_GEMM_SPLITS=n their K split;
+  // ORCA_HIP_GEMM_SMALL_TILES=0 keeps them on tiles of 128.
   bool gemm_generic_only = false;
-  int gemm_tile_bn = 0;
+  int gemm_generic_bn = 0;
+  int gemm_tile = 0;
   int gemm_splits = 0;
   // ORCA_HIP_GEMM_NARROW=0 keeps products with N <= 16 (or K <= 16 against B^T) on the tiled kernels.
   bool gemm_narrow = true;

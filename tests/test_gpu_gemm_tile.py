@@ -18,22 +18,28 @@ from tests.util import int_matrix
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module", params=["16/1", "32/1", "64/1", "128/1", "16/2", "32/3", "64/2", "128/3"])
-def tctx(request):
-    """A context whose products take one tile (and K split)."""
+def context(**switches):
+    """A context created under ORCA_HIP_GEMM_<name>=<value>."""
     from orcaml_amd.device import Context
 
-    tile, splits = request.param.split("/")
-    old = {k: os.environ.get(k) for k in ("ORCA_HIP_GEMM_TILE", "ORCA_HIP_GEMM_SPLITS")}
-    os.environ.update(ORCA_HIP_GEMM_TILE=tile, ORCA_HIP_GEMM_SPLITS=splits)
+    names = {f"ORCA_HIP_GEMM_{k}": v for k, v in switches.items()}
+    old = {k: os.environ.get(k) for k in names}
+    os.environ.update(names)
     try:
-        c = Context(0)
+        return Context(0)
     finally:
         for k, v in old.items():
             if v is None:
                 del os.environ[k]
             else:
                 os.environ[k] = v
+
+
+@pytest.fixture(scope="module", params=["16/1", "32/1", "64/1", "128/1", "16/2", "32/3", "64/2", "128/3"])
+def tctx(request):
+    """A context whose products take one tile (and K split)."""
+    tile, splits = request.param.split("/")
+    c = context(TILE=tile, SPLITS=splits)
     yield c
     c.close()
 
@@ -193,3 +199,24 @@ def test_more_rows_than_grid_rows_of_small_tiles(ctx):
     a, b, c = ctx.upload(A), ctx.upload(B), ctx.alloc(A.shape[0] * 80)
     _lib.call("orca_hip_gemm", ctx.handle, 0, 0, A.shape[0], 20, 32, a.ptr, 32, b.ptr, 20, c.ptr, 20, None)
     np.testing.assert_array_equal(c.download(count=A.shape[0] * 20).reshape(-1, 20), A @ B)
+
+
+@pytest.mark.parametrize("switches,kernel", [
+    ({"TILE": "16"}, "gemm_nn_t16"), ({"TILE": "128"}, "gemm_nn_pipe"), ({"SMALL_TILES": "0"}, "gemm_nn_pipe"),
+    # the generic kernel's tile, and values that name no tile: the cost rule's choice for the others
+    ({"TILE": "128x64"}, "gemm_nn_t32"), ({"TILE": "128x128"}, "gemm_nn_t32"), ({"TILE": "64abc"}, "gemm_nn_t32"),
+    ({"TILE": "128x64", "FAST": "0"}, "gemm_nn"), ({"TILE": "128x128", "FAST": "0"}, "gemm_nn")])
+def test_tile_switches(switches, kernel):
+    ctx = context(**switches)
+    if ctx.prof_report()["num_cus"] != 256:
+        pytest.skip("tile counts chosen for 256 compute units")
+    rng = np.random.default_rng(1)
+    A, B = int_matrix(rng, (256, 1024)), int_matrix(rng, (1024, 1024))
+    ctx.prof_reset()
+    ctx.prof_enable(True)
+    got = product(ctx, False, False, A, B)[0]
+    ctx.prof_enable(False)
+    np.testing.assert_array_equal(got, (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32))
+    names = {k["name"].split()[0] for k in ctx.prof_report()["kernels"]}
+    assert kernel in names, names
+    ctx.close()
