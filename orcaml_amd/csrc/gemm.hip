@@ -1504,7 +1504,8 @@ void choose_tile(orca_hip_ctx* ctx, GemmPlan& g, bool trans_a, bool trans_b, siz
     const size_t tiles = ((M + t - 1) / t) * ((N + t - 1) / t) * batch, slabs = (K + f.slab_k - 1) / f.slab_k;
     for (int j = 0; j < 3; ++j) {
       size_t s = j == 0 ? 1 : std::min<size_t>(std::min<size_t>((size_t)j * target / tiles, slabs / 2), 64);
-      if (ctx->gemm_splits) s = std::min<size_t>((size_t)ctx->gemm_splits, slabs);
+      // a forced split: grid z, one layer per entry and chunk, ends at 65535
+      if (ctx->gemm_splits) s = std::min<size_t>({(size_t)ctx->gemm_splits, slabs, std::max<size_t>(1, 65535 / batch)});
       if (s == 0 || (j > 0 && s == 1)) continue;
       const size_t per = (slabs + s - 1) / s;
       s = (slabs + per - 1) / per;

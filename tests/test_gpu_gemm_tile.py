@@ -153,6 +153,21 @@ def test_every_tile_batched(tctx, batch, M, N, K):
         np.testing.assert_array_equal(got, want)
 
 
+def test_forced_split_of_many_entries_stays_within_the_grid():
+    """64 chunks of each of 1100 entries would be 70400 layers of the grid."""
+    from orcaml_amd.backend import HipBackend
+
+    ctx = context(TILE="64", SPLITS="64")
+    be = HipBackend(ctx)
+    rng = np.random.default_rng(2)
+    A, B = int_matrix(rng, (1100, 4, 4096), -1, 2), int_matrix(rng, (1100, 4096, 4), -1, 2)
+    a, b = be.from_f32_slice(A.shape, A), be.from_f32_slice(B.shape, B)
+    got = be.to_f32_vec(be.matmul(a, b, A.shape, B.shape)).reshape(1100, 4, 4)
+    np.testing.assert_array_equal(got, A @ B)
+    del a, b, be
+    ctx.close()
+
+
 @pytest.mark.parametrize("batch,m,k,n", [(3, 33, 20, 65), (5, 197, 64, 197), (7, 70, 300, 40), (2, 16, 5, 18), (9, 130, 70, 31)])
 def test_batched_tiles_in_any_number(ctx, batch, m, k, n):
     """Tile counts that are no multiple of the eight XCDs, each operand transposed in turn."""
