@@ -135,7 +135,8 @@ def test_every_tile_epilogues_and_column_sum_bits(tctx, M, N, K):
         np.testing.assert_array_equal(p, kept)
 
 
-@pytest.mark.parametrize("batch,M,N,K", [(5, 40, 24, 70), (3, 197, 197, 64), (260, 9, 8, 33)])
+@pytest.mark.parametrize("batch,M,N,K", [(5, 40, 24, 70), (3, 197, 197, 64), (260, 9, 8, 33),
+                                           (3, 130, 70, 130)])  # 18 64-tiles, six an entry, in three slabs
 def test_every_tile_batched(tctx, batch, M, N, K):
     from orcaml_amd.backend import HipBackend
 
@@ -168,11 +169,15 @@ def test_forced_split_of_many_entries_stays_within_the_grid():
     ctx.close()
 
 
-@pytest.mark.parametrize("batch,m,k,n", [(3, 33, 20, 65), (5, 197, 64, 197), (7, 70, 300, 40), (2, 16, 5, 18), (9, 130, 70, 31)])
+@pytest.mark.parametrize("batch,m,k,n", [(3, 33, 20, 65), (5, 197, 64, 197), (7, 70, 300, 40), (2, 16, 5, 18), (9, 130, 70, 31),
+                                           (13, 330, 64, 330), (21, 260, 64, 260)])
 def test_batched_tiles_in_any_number(ctx, batch, m, k, n):
-    """Tile counts that are no multiple of the eight XCDs, each operand transposed in turn."""
+    """Tile counts that are no multiple of the eight XCDs, each operand transposed in turn; the last two
+    on 64-tiles, 468 and 525 of them, whose order follows the XCDs."""
     from orcaml_amd.backend import HipBackend
 
+    ctx.prof_reset()
+    ctx.prof_enable(True)
     rng = np.random.default_rng(batch * m + n)
     be = HipBackend(ctx)
     A, B = int_matrix(rng, (batch, m, k), -3, 4), int_matrix(rng, (batch, k, n), -3, 4)
@@ -183,6 +188,9 @@ def test_batched_tiles_in_any_number(ctx, batch, m, k, n):
         b = be.transpose(b, (batch, n, k), 1, 2) if tb else b
         out = np.asarray(be.to_f32_vec(be.matmul(a, b, (batch, m, k), (batch, k, n)))).reshape(batch, m, n)
         np.testing.assert_array_equal(out, A @ B)
+    ctx.prof_enable(False)
+    if m > 250 and ctx.prof_report()["num_cus"] == 256:
+        assert all("_t64" in name["name"] for name in ctx.prof_report()["kernels"] if name["name"].startswith("gemm_"))
 
 
 @pytest.mark.parametrize("ta,M,N,K,tiles", [
@@ -208,11 +216,18 @@ def test_tile_of_lopsided_products(ctx, ta, M, N, K, tiles):
 
 
 def test_more_rows_than_grid_rows_of_small_tiles(ctx):
-    """2^21 + 3 rows: 32-row tiles, the cheapest for this width, would need 65537 grid rows."""
+    """2^21 + 3 rows: 32-row tiles, the cheapest for this width and a K of one of their slabs and two of
+    the 64-tiles', would need 65537 grid rows; 100 rows less and they are taken."""
     rng = np.random.default_rng(5)
-    A, B = int_matrix(rng, ((1 << 21) + 3, 32), -2, 3), int_matrix(rng, (32, 20), -2, 3)
+    A, B = int_matrix(rng, ((1 << 21) + 3, 68), -2, 3), int_matrix(rng, (68, 20), -2, 3)
     a, b, c = ctx.upload(A), ctx.upload(B), ctx.alloc(A.shape[0] * 80)
-    _lib.call("orca_hip_gemm", ctx.handle, 0, 0, A.shape[0], 20, 32, a.ptr, 32, b.ptr, 20, c.ptr, 20, None)
+    for rows, tile in ((A.shape[0] - 100, "_t32"), (A.shape[0], "_t64")):
+        ctx.prof_reset()
+        ctx.prof_enable(True)
+        _lib.call("orca_hip_gemm", ctx.handle, 0, 0, rows, 20, 68, a.ptr, 68, b.ptr, 20, c.ptr, 20, None)
+        ctx.prof_enable(False)
+        if ctx.prof_report()["num_cus"] == 256:
+            assert any(f"gemm_nn{tile}_ua" in k["name"] for k in ctx.prof_report()["kernels"])
     np.testing.assert_array_equal(c.download(count=A.shape[0] * 20).reshape(-1, 20), A @ B)
 
 

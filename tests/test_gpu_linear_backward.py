@@ -1,5 +1,5 @@
 """A hidden layer's two backward products from one grid (the trainer's small layers): every
-gradient against an fp64 backward pass, at sizes that take the different tile pairs, aligned and
+gradient against an fp64 backward pass, at sizes that take each of the tile pairs, aligned and
 odd, with the bias gradient from the grid's own blocks and from the head."""
 from __future__ import annotations
 
@@ -31,10 +31,16 @@ def backward64(dims, params, x, labels):
     return grads
 
 
-@pytest.mark.parametrize("dims,batch", [
-    ((64, 128, 128, 10), 64), ((24, 19, 21, 5), 3), ((100, 1024, 1024, 10), 256), ((50, 1001, 333, 26), 200),
-    ((20, 257, 129, 33, 20), 65), ((16, 300, 40, 64, 18), 130), ((32, 900, 1100, 10), 250), ((8, 36, 2000, 40), 64)])
-def test_gradients_of_paired_products(ctx, dims, batch):
+@pytest.mark.parametrize("dims,batch,pairs", [
+    ((64, 128, 128, 10), 64, {"t16_t16"}), ((24, 19, 21, 5), 3, {"t16_t16_ua"}),
+    ((100, 1024, 1024, 10), 256, {"t32_t64"}), ((50, 1001, 333, 26), 200, {"t32_t32_ua", "t32_t16_ua"}),
+    ((20, 257, 129, 33, 20), 65, {"t16_t16_ua"}), ((16, 300, 40, 64, 18), 130, {"t16_t16_ua"}),
+    ((32, 900, 1100, 10), 250, {"t32_t64_ua"}), ((8, 36, 2000, 40), 64, {"t16_t16", "t32_t32"}),
+    ((20, 1933, 680, 10), 568, {"t64_t64_ua"}), ((24, 1308, 252, 10), 576, {"t64_t64"}),
+    ((20, 616, 96, 10), 8, {"t32_t16"})])
+def test_gradients_of_paired_products(ctx, dims, batch, pairs):
+    if ctx.prof_report()["num_cus"] != 256:
+        pytest.skip("tile counts chosen for 256 compute units")
     rng = np.random.default_rng(sum(dims) + batch)
     # small integers scaled by powers of two: the forward pass is exact, so the ReLU masks are
     params = []
@@ -50,7 +56,7 @@ def test_gradients_of_paired_products(ctx, dims, batch):
     tr.step()
     ctx.prof_enable(False)
     names = {k["name"].split()[0] for k in ctx.prof_report()["kernels"]}
-    assert any(n.startswith("gemm_linear_bw_") for n in names), names
+    assert {n.replace("gemm_linear_bw_", "") for n in names if n.startswith("gemm_linear_bw_")} == pairs, names
     for i, (got, want) in enumerate(zip(tr.grads(), backward64(dims, params, x, labels))):
         # f32 sums of at most max(batch, width) terms per layer, the logits exact
         err = np.linalg.norm(got - want) / max(np.linalg.norm(want), 1e-30)
