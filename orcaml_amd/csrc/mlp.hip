@@ -13,12 +13,15 @@
 //   backward  L GEMMs dW = A^T dZ with the bias column sum fused in, and
 //             L-1 GEMMs dZ_prev = (dZ W^T) * [H > 0] with the mask fused in
 //   update    one AdamW or SGD pass over the whole parameter arena.
+// A model without a second stream (below) whose layer 0 runs unsplit on small
+// tiles has the whole update in the launch of that layer's dW, and its hidden
+// layers' dW and dZ_prev from one grid where that is estimated faster (gemm.hip).
 // When the last layer has at most 16 outputs (a classifier), its three
 // products and the loss are HBM-bound rather than GEMM-shaped; they run as
 // the two fused head kernels instead (forward + loss, and backward), each
 // streaming the layer's input once.  ORCA_HIP_FUSED_HEAD=0 at creation keeps
 // the GEMM + softmax-CE path, ORCA_HIP_OVERLAP_UPDATE=0 runs the whole update
-// on the context stream after the backward (A/B comparisons).
+// as a pass of its own on the context stream after the backward (A/B comparisons).
 // With AdamW and a side stream the parameters have two arenas, P and P_next:
 // the update reads P and writes P_next, and they swap after each step.  The
 // update of layers >= 1 then starts right after dW of layer 1, beside layer
@@ -58,6 +61,7 @@ struct orca_hip_mlp {
   float* loss = nullptr;
   int64_t* correct = nullptr;
   int32_t* preds = nullptr;
+  bool update_in_dw0 = false;  // the update may run in the launch of layer 0's dW
   std::vector<void*> owned;
   bool have_batch = false;
   bool fused_head = false;
@@ -245,7 +249,7 @@ void step_body(orca_hip_mlp* m, const AdamWScalars* kdev) {
       continue;
     }
     // Small first layers: the whole update in the launch of layer 0's weight gradient.
-    if (l == 0 && !m->side && m->shard_count == 1) {
+    if (l == 0 && m->update_in_dw0 && m->shard_count == 1) {
       ArenaUpdate u{};
       u.adamw = m->opt.kind == 1;
       u.P = m->P;
@@ -425,8 +429,10 @@ int orca_hip_mlp_create(orca_hip_ctx* ctx, const size_t* dims, size_t n_layers, 
     // The fork / join costs more than it hides unless the overlapped update is
     // large (measured: it slows the 784-128-128-10 and 784-1024-1024-10 steps).
     const char* ov = std::getenv("ORCA_HIP_OVERLAP_UPDATE");
+    const bool own_pass = ov && ov[0] == '0';
     const size_t overlapped = n_layers > 1 ? o - m->off[2] : 0;
-    if (overlapped >= kMinOverlapParams && !(ov && ov[0] == '0')) {
+    m->update_in_dw0 = overlapped < kMinOverlapParams && !own_pass;
+    if (overlapped >= kMinOverlapParams && !own_pass) {
       ORCA_HIP_CHECK(hipStreamCreateWithFlags(&m->side, hipStreamNonBlocking));
       ORCA_HIP_CHECK(hipEventCreateWithFlags(&m->fork, kStreamEventFlags));
       ORCA_HIP_CHECK(hipEventCreateWithFlags(&m->join, kStreamEventFlags));

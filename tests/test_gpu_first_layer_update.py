@@ -56,3 +56,31 @@ def test_update_beside_the_first_weight_gradient(ctx, kind, dims, batch):
                 for got, w in zip(tr.moments(which), state):
                     np.testing.assert_array_equal(got, w)
     tr.close()
+
+
+@pytest.mark.parametrize("kind", ["sgd", "adamw"])
+def test_update_as_a_pass_of_its_own(ctx, kind, monkeypatch):
+    """ORCA_HIP_OVERLAP_UPDATE=0: no update in the weight gradient's launch, the same bits."""
+    dims, batch, got = (100, 130, 64, 10), 48, []
+    rng = np.random.default_rng(9)
+    params = []
+    for i, o in zip(dims[:-1], dims[1:]):
+        params += [(rng.standard_normal((i, o)) / math.sqrt(i)).astype(f32), rng.standard_normal((1, o)).astype(f32)]
+    x, labels = rng.random((batch, dims[0]), dtype=f32), rng.integers(0, 10, batch).astype(np.int32)
+    for own in (False, True):
+        if own:
+            monkeypatch.setenv("ORCA_HIP_OVERLAP_UPDATE", "0")
+        tr = MLPTrainer(ctx, dims, batch, kind=kind, lr=1e-2)
+        tr.set_params(params)
+        tr.set_batch(x, labels=labels)
+        ctx.prof_reset()
+        ctx.prof_enable(True)
+        for _ in range(3):
+            tr.step()
+        ctx.prof_enable(False)
+        names = {k["name"].split()[0] for k in ctx.prof_report()["kernels"]}
+        assert any(n.endswith("_update") for n in names) != own and (kind in names) == own, names
+        got.append(tr.params())
+        tr.close()
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
