@@ -12,7 +12,7 @@
 // block (4 wave64s as 2 x 2) owns a 128 x 128 tile of C and each wave 2 x 2 MFMA
 // 32x32 blocks; K advances in slabs of 32 held in double-buffered LDS (72 KiB,
 // so two blocks fit in one CU's 160 KiB), one barrier per slab.  Products that
-// do not take tiles of 64, 32 or 16 (gemm_tile.hpp), and choose_tile says which
+// do not fill it take tiles of 64, 32 or 16 (gemm_tile.hpp); choose_tile says which
 // and how K splits.  The generic kernel (128 x 128 or 128 x 64 tiles, every load
 // checked) is left for operands of 4 GiB and more and for the few shapes with
 // less than four floats in a row.

@@ -92,7 +92,8 @@ __device__ __forceinline__ void tile_product(const GemmParams& p, int bx, int by
             const float* s = smem + decltype(buf)::value * SLAB + tid;
             const int rows = min(KS, p.K - t * KS);
             // 64 rows' reads ahead of their adds (rows past K are zero): the chain of adds
-            // is what takes the time, about 3 ns a row
+            // is what takes the time, 4.6 to 5.5 ns a row with the loads (X^T dY of 16 x 112 x 1288:
+            // 9.3 us beside a product of 6.1), 6.6 where T is 32 or 64
             for (int k = 0; k < rows; k += 64) {
               float v[64];
 #pragma unroll
