@@ -206,3 +206,29 @@ def test_trainer_fused_head_equals_gemm_head(ctx, monkeypatch, workload):
         assert_close_scaled(a, b, rtol=1e-3, what=f"grad {i}")
     for i, (a, b) in enumerate(zip(p1, p0)):
         assert_close(a, b, what=f"param {i}")
+
+
+@pytest.mark.parametrize("B", [5, 1030])
+@pytest.mark.parametrize("K", [64, 4064, 4096, 4100])
+def test_training_step_finishes_the_loss_on_every_grid(ctx, B, K):
+    """A step's backward kernel adds up the forward's row terms: in a block of its own while a CU is
+    free for it (4 and 254 panels of 16 columns on 256 CUs), in block 0 from 256 panels on."""
+    rng = np.random.default_rng(B + K)
+    dims = [12, K, 10]
+    params = []
+    for i, o in zip(dims[:-1], dims[1:]):
+        params += [int_matrix(rng, (i, o), -1, 2), int_matrix(rng, (1, o), -2, 3)]
+    params[2] *= np.float32(2.0 ** -6)
+    x, labels = int_matrix(rng, (B, 12), 0, 3), rng.integers(0, 10, B).astype(np.int32)
+    tr = MLPTrainer(ctx, dims, B, kind="sgd", lr=0.0)
+    tr.set_params(params)
+    tr.set_batch(x, labels=labels)
+    tr.step()
+    loss, correct = tr.metrics()
+    # integers over 64: the logits are exact in any order
+    z = np.maximum(x @ params[0] + params[1], 0).astype(np.float64) @ params[2] + params[3]
+    z -= z.max(1, keepdims=True)
+    want = (np.log(np.exp(z).sum(1)) - z[np.arange(B), labels]).mean()
+    assert abs(loss - want) <= 1e-6 * max(1.0, want)
+    assert correct == int((np.argmax(tr.logits(), 1) == labels).sum())
+    tr.close()
