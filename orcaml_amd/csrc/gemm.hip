@@ -1457,8 +1457,10 @@ std::string kernel_name(const GemmPlan& g, bool ta, bool tb) {
 //   3 us + r (per block + slabs per block * per slab)
 // and a split adds its reduce launch, 3 us and the partial sums at 5 TB/s.  Blocks of one slab
 // run four to a CU and hide most of each other's loads and stores, so their rounds up to the
-// fourth cost `beside` of the first and the others `after`; a 64-tile whose K ends in the slab's first half multiplies half
-// (X W of 2290 x 1128 x 10: 9.9 us on tiles of 128, 7.0 on tiles of 64).  X^T dY is priced with
+// fourth cost `beside` of the first and the others `after`; a 64-tile whose K ends in the slab's
+// first half multiplies half (X W of 2290 x 1128 x 10: 9.9 us on tiles of 128, 7.0 on tiles of 64).
+// Batched blocks overlap little: 0.15 us less a round (96 x [197 x 32] x [32 x 197]: 11.8 us on
+// tiles of 128, 14.2 on the 64-tiles that the single products' terms would choose).  X^T dY is priced with
 // its bias gradient (the plan must not depend on whether that is asked for, so that the
 // product's bits do not): a chain of adds beside the small tiles' product, 5 ns a row beside
 // tiles of 16 and 6.6 beside the others, 0.19 us a slab folded into the 128 tiles, a launch of
@@ -1486,7 +1488,7 @@ struct TileForm {
 };
 constexpr TileForm kTileForms[4] = {{16, 256, 0.4, 0.5, 0.3, 0.7, 5.0, {{0.50, 0.60, 0.95}, {0.55, 0.70, 1.05}}},
                                     {32, 128, 0.5, 0.3, 0.55, 0.7, 6.6, {{0.64, 0.68, 0.85}, {0.68, 0.90, 0.95}}},
-                                    {64, 64, 1.0, 0.15, 0.5, 0.5, 6.6, {{1.06, 1.06, 1.13}, {1.06, 1.10, 1.25}}},
+                                    {64, 64, 1.0, 0.15, 0.5, 0.9, 6.6, {{1.06, 1.06, 1.13}, {1.06, 1.10, 1.25}}},
                                     {128, BK, 3.0, 0.0, 1.0, 1.0, 0.0, {{1.82, 1.82, 1.82}, {1.84, 1.84, 1.84}}}};
 // The chain of adds of a column sum beside small tiles, us for k rows.
 constexpr double colsum_chain_us(const TileForm& f, size_t k) { return 3.0 + 1e-3 * f.colsum_ns * (double)k; }
@@ -1510,10 +1512,12 @@ void choose_tile(orca_hip_ctx* ctx, GemmPlan& g, bool trans_a, bool trans_b, siz
       const size_t per = (slabs + s - 1) / s;
       s = (slabs + per - 1) / per;
       const double rounds = (double)((tiles * s + target - 1) / target);
-      const double slab = f.slab_us[g.ua ? 1 : 0][mn_fast] * (f.tile == 64 && K <= 32 ? 0.5 : 1.0);
-      const double block = f.block_us + (double)per * slab;
+      const bool half = batch == 1 && f.tile == 64 && K <= 32;
+      const double block = f.block_us + (double)per * f.slab_us[g.ua ? 1 : 0][mn_fast] * (half ? 0.5 : 1.0);
       double product = 3.0;
-      if (slabs == 1 && f.tile < 128)
+      if (slabs == 1 && f.tile < 128 && batch > 1)
+        product += (block - 0.15) * rounds;
+      else if (slabs == 1 && f.tile < 128)
         product += block * (1.0 + f.beside * (std::min(rounds, 4.0) - 1.0) + f.after * std::max(rounds - 4.0, 0.0)) - f.one_slab_us;
       else
         product += block * rounds;
@@ -2106,7 +2110,7 @@ void gemm_launch(orca_hip_ctx* ctx, bool trans_a, bool trans_b, size_t M, size_t
       bound = bind;
       if (plan.tile == 16) TILE_LAUNCH(16);
       else if (plan.tile == 32) TILE_LAUNCH(32);
-      else if (batch > 1) {
+      else if (batch > 1 && epi.kind == ORCA_HIP_EPI_NONE) {
         if (plan.ua && K <= 64) TILE_BATCH_LAUNCH(true, true);
         else if (plan.ua) TILE_BATCH_LAUNCH(true, false);
         else if (K <= 64) TILE_BATCH_LAUNCH(false, true);

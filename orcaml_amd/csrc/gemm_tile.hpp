@@ -259,12 +259,14 @@ __global__ void __launch_bounds__(256, ONE ? 4 : 2) gemm_tile_kernel(GemmParams 
 // 44.4.  (Entries of smaller tiles: no difference.  A single product keeps the dispatch order,
 // in which an XCD has every eighth column of tiles with all of its rows, and a kernel without
 // this arithmetic: as a branch of one kernel it cost single products 0.2 us a launch.)
+// Batched products have no epilogue: without the others' code 46.8 -> 43.0 us.
 template <bool TA, bool TB, bool UA, bool ONE>
 __global__ void __launch_bounds__(256, ONE ? 4 : 2) gemm_tile_batch_kernel(GemmParams p) {
   __shared__ __attribute__((aligned(16))) float smem[(ONE ? 1 : 2) * tile_slab_floats<64, TA, TB, UA>()];
   const uint32_t nx = gridDim.x, per = nx * gridDim.y, blocks = per * gridDim.z;
   const uint32_t l = blockIdx.x + nx * blockIdx.y + per * blockIdx.z, xcd = l % 8;
   const uint32_t id = xcd * (blocks / 8) + min(xcd, blocks % 8) + l / 8, in = id % per;
+  p.epi = ORCA_HIP_EPI_NONE;
   tile_product<64, TA, TB, UA, ONE>(p, in % nx, in / nx, id / per, smem);
 }
 

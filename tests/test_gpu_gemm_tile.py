@@ -136,7 +136,8 @@ def test_every_tile_epilogues_and_column_sum_bits(tctx, M, N, K):
 
 
 @pytest.mark.parametrize("batch,M,N,K", [(5, 40, 24, 70), (3, 197, 197, 64), (260, 9, 8, 33),
-                                           (3, 130, 70, 130)])  # 18 64-tiles, six an entry, in three slabs
+                                           (3, 130, 70, 130),  # 18 64-tiles, six an entry, in three slabs
+                                           (3, 70, 66, 32)])  # half of a slab
 def test_every_tile_batched(tctx, batch, M, N, K):
     from orcaml_amd.backend import HipBackend
 
