@@ -1793,7 +1793,7 @@ bool narrow_linear_backward(orca_hip_ctx* ctx, const float* H, size_t B, size_t 
 }  // namespace
 
 // dX = (dY W^T) masked and dW = X^T dY (+ column sums) in one launch, when the estimate says
-// that pays: the pair's time is its blocks' work spread over the CUs plus half a block's (or
+// that pays: the pair's time is its blocks' work spread over the CUs plus 0.3 of a block's (or
 // one block's, if they all start at once), against the two plans' own times and the gap
 // between two launches.  784-1024-1024-10, 256 rows: 9.9 + 9.1 -> 15.3 us.  False (nothing
 // launched) when the two run apart.
@@ -1810,19 +1810,32 @@ bool gemm_linear_backward(orca_hip_ctx* ctx, size_t B, size_t K, size_t N, const
   static constexpr Pair pairs[5] = {{0, 0}, {1, 0}, {1, 1}, {1, 2}, {2, 2}};  // of kTileForms
   const double cus = (double)ctx->num_cus;
   auto tiles = [](size_t m, size_t n, size_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
-  auto block = [&](const TileForm& f, int mn_fast, size_t k) {
-    return f.block_us + (double)((k + f.slab_k - 1) / f.slab_k) * f.slab_us[ua][mn_fast];
+  // In this kernel a block takes so much more, and its slabs this share, of what it takes alone
+  // (fits to HIP-event times of each pair for 252 layers, 8 to 1024 rows: the choices take 0.8 %
+  // more than the best pairs in the geometric mean, 3.4 % without these terms; 200 x 333 x 26:
+  // 6.6 us on tiles of 32 and 16, 5.3 on tiles of 16).
+  struct PairCost {
+    double x_us, x_slab, w_us, w_slab;
+  };
+  static constexpr PairCost cost[3] = {{0.3, 0.7, 0.0, 0.6}, {1.2, 0.8, 1.0, 0.8}, {0.0, 1.0, 1.1, 1.3}};
+  auto block = [&](const TileForm& f, double more_us, double slab, int mn_fast, size_t k) {
+    return f.block_us + more_us + (double)((k + f.slab_k - 1) / f.slab_k) * f.slab_us[ua][mn_fast] * slab;
   };
   int best = -1;
-  double best_us = px.us + pw.us + 1.0;
+  // Apart: both plans and a gap of 1 us between them, whose work in the pair's terms is 1 / 0.85
+  // of theirs (three of the 252 layers then take the slower way, by 5 to 15 %).
+  double best_us = 3.0 + (px.us + pw.us - 2.0) / 0.85, best_products = best_us;
   for (int i = 0; i < 5; ++i) {
     const TileForm &fx = kTileForms[pairs[i].x], &fw = kTileForms[pairs[i].w];
-    const double bx = block(fx, 0, N), bw = block(fw, 2, B);
+    const PairCost &cx = cost[pairs[i].x], &cw = cost[pairs[i].w];
+    const double bx = block(fx, cx.x_us, cx.x_slab, 0, N), bw = block(fw, cw.w_us, cw.w_slab, 2, B);
     const double nx = (double)tiles(B, K, (size_t)fx.tile), nw = (double)tiles(K, N, (size_t)fw.tile);
-    const double longest = std::max(bx, bw), spread = (nx * bx + nw * bw) / cus + 0.5 * longest;
-    const double us = std::max(3.0 + (nx + nw <= cus ? longest : std::max(longest, spread)), colsum ? colsum_chain_us(fw, B) : 0.0);
-    if (us < best_us) {
+    const double longest = std::max(bx, bw), spread = (nx * bx + nw * bw) / cus + 0.3 * longest;
+    const double products = 3.0 + (nx + nw <= cus ? longest : std::max(longest, spread));
+    const double us = std::max(products, colsum ? colsum_chain_us(fw, B) : 0.0);
+    if (us < best_us || (us == best_us && products < best_products)) {
       best_us = us;
+      best_products = products;
       best = i;
     }
   }

@@ -33,11 +33,11 @@ def backward64(dims, params, x, labels):
 
 @pytest.mark.parametrize("dims,batch,pairs", [
     ((64, 128, 128, 10), 64, {"t16_t16"}), ((24, 19, 21, 5), 3, {"t16_t16_ua"}),
-    ((100, 1024, 1024, 10), 256, {"t32_t64"}), ((50, 1001, 333, 26), 200, {"t32_t32_ua", "t32_t16_ua"}),
+    ((100, 1024, 1024, 10), 256, {"t32_t64"}), ((50, 1001, 333, 26), 200, {"t32_t32_ua", "t16_t16_ua"}),
     ((20, 257, 129, 33, 20), 65, {"t16_t16_ua"}), ((16, 300, 40, 64, 18), 130, {"t16_t16_ua"}),
     ((32, 900, 1100, 10), 250, {"t32_t64_ua"}), ((8, 36, 2000, 40), 64, {"t16_t16", "t32_t32"}),
     ((20, 1933, 680, 10), 568, {"t64_t64_ua"}), ((24, 1308, 252, 10), 576, {"t64_t64"}),
-    ((20, 616, 96, 10), 8, {"t32_t16"})])
+    ((20, 904, 40, 10), 640, {"t32_t16"}), ((20, 167, 121, 10), 674, {"t32_t16_ua"})])
 def test_gradients_of_paired_products(ctx, dims, batch, pairs):
     if ctx.prof_report()["num_cus"] != 256:
         pytest.skip("tile counts chosen for 256 compute units")
