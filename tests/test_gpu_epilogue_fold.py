@@ -32,12 +32,15 @@ def gemm_pre(ctx, A_, B_, bias):
 
 
 @pytest.mark.parametrize("M,N,K", [
-    (256, 384, 160),    # pipelined 128 x 128 kernel
-    (260, 196, 164),    # pipelined, edge tiles
+    (256, 384, 160),    # 16 x 16 tiles
+    (260, 196, 164),    # 16 x 16 tiles, edges
+    (2048, 2048, 160),  # pipelined 128 x 128 kernel
+    (2044, 2040, 164),  # pipelined, edge tiles
     (256, 1024, 784),   # 32 x 32 tiles
     (1024, 1024, 256),  # 64 x 64 tiles
     (128, 256, 3076),   # split K: the epilogue runs in the float4 reduce
-    (130, 70, 33),      # generic kernel, unaligned
+    (130, 70, 33),      # 16 x 16 tiles, unaligned
+    (130, 70, 3),       # generic kernel
     (129, 1029, 1021),  # 32 x 32 tiles, ragged
     (64, 13, 2050),     # N <= 16 stays on the tiles (split K, scalar reduce)
 ])
@@ -60,10 +63,11 @@ def test_bias_relu_pre_epilogue_matches_composed_ops(ctx, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [
-    (256, 384, 160),    # pipelined 128 x 128 kernel (B^T)
+    (256, 384, 160),    # 16 x 16 tiles (B^T)
+    (2044, 2040, 164),  # pipelined 128 x 128 kernel (B^T), edge tiles
     (256, 1024, 1024),  # 32 x 32 tiles (B^T)
     (128, 256, 3076),   # split K: the float4 reduce
-    (130, 70, 33),      # generic kernel, unaligned: the scalar reduce or the tile store
+    (130, 70, 33),      # 16 x 16 tiles, unaligned
     (1024, 4096, 10),   # narrow K against B^T
     (33, 1001, 3),
 ])
@@ -195,7 +199,7 @@ def test_relu_backward_on_a_held_product(ctx):
 
 
 @pytest.mark.parametrize("M,N,K", [(256, 384, 160), (256, 1024, 1024), (128, 256, 3076), (130, 70, 33),
-                                   (1024, 10, 4096), (1024, 4096, 10), (64, 13, 2050)])
+                                   (2044, 2040, 164), (130, 70, 3), (1024, 10, 4096), (1024, 4096, 10), (64, 13, 2050)])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False)])
 def test_products_never_hold_negative_zero(ctx, M, N, K, ta, tb):
     """Every GEMM path (pipelined, small tiles, split K, generic, narrow) returns +0 where all

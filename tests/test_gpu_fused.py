@@ -54,15 +54,17 @@ def assert_gemm_error_bound(got, A, B):
 
 
 GEMM_SHAPES = [
-    # generic kernel (a dimension not a multiple of 4, or N / K = 10 as in the output layer)
+    # generic kernel (K = 1), unaligned small tiles, N / K = 10 as in the output layer
     (1, 1, 1), (130, 70, 33), (257, 129, 1000), (1024, 10, 4096), (1024, 4096, 10),
-    # pipelined kernel, edge tiles and partial K slabs (K = 784 as in the input layer)
+    # small tiles, edges and partial K slabs (K = 784 as in the input layer)
     (64, 128, 784), (784, 384, 1024), (96, 16, 4), (4, 8, 12), (132, 260, 36), (200, 300, 152),
-    # pipelined kernel, tile-aligned: 1..5 and 32 slabs, and split-K launches
+    # tile-aligned, one slab to many, and split-K launches
     (128, 128, 32), (256, 128, 64), (128, 256, 96), (256, 256, 128), (384, 128, 160), (256, 384, 1024),
     (128, 128, 4096), (128, 256, 3076),
-    # 128 tiles of 128 x 128: half of MI355X's 256 CUs, so K splits in two
-    (1024, 2048, 128)]
+    # 128 tiles of 128 x 128: half of MI355X's 256 CUs
+    (1024, 2048, 128),
+    # pipelined kernel, whole and edge tiles
+    (2048, 2048, 160), (2044, 2040, 164)]
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
@@ -186,10 +188,12 @@ def test_gemm_small_tiles_exact_on_integers(ctx, ta, tb, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(200, 300, 150), (200, 300, 152), (256, 384, 128), (128, 256, 1024),
-                                   (130, 70, 1000), (1024, 2048, 128)])
+                                   (130, 70, 1000), (1024, 2048, 128), (2048, 2048, 160), (2044, 2040, 164),
+                                   (200, 300, 2)])
 def test_gemm_epilogues_match_composed_ops(ctx, M, N, K):
-    """Generic kernel (K = 150), pipelined kernel with edge tiles (152) and aligned (128); split-K
-    launches whose epilogue runs in the float4 reduce (N = 256, 2048) or the scalar one (N = 70)."""
+    """Small tiles, aligned and not, the pipelined kernel's whole and edge tiles, the generic kernel
+    (K = 2); split-K launches whose epilogue runs in the float4 reduce (N = 256) or the scalar one
+    (N = 70)."""
     rng = np.random.default_rng(5)
     A = rng.standard_normal((M, K)).astype(np.float32)
     B = rng.standard_normal((K, N)).astype(np.float32)

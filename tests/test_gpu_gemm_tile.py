@@ -109,7 +109,7 @@ def test_every_tile_exact_on_integers(tctx, M, N, K):
                     np.testing.assert_array_equal(got[1], sums, err_msg=f"{ta} {tb} {pad} {shift}")
 
 
-@pytest.mark.parametrize("M,N,K", [(33, 65, 257), (128, 64, 512), (130, 70, 300)])
+@pytest.mark.parametrize("M,N,K", [(33, 65, 257), (128, 64, 512), (130, 70, 300), (128, 256, 96)])
 def test_every_tile_epilogues_and_column_sum_bits(tctx, M, N, K):
     """Real data: each epilogue is the composed ops on the tile's own product, bit for bit, and the
     column sum has the bits of sum_to_shape."""

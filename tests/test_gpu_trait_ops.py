@@ -247,7 +247,7 @@ def test_composed_step_mlp784_128_on_hip(hb, kind, steps):
 def test_matmul_colsum_equals_matmul_and_sum_to_shape(hb, M, K, N, view):
     """orca_hip_matmul_colsum (via a pending sum_to_shape consumed by matmul): the product bit
     for bit as matmul, the column sum bit for bit as the oracle's sum_to_shape loop -- folded
-    into the product (pipelined or generic kernel) or, when K is split, in its own pass."""
+    into the product or, when K is split, in its own pass."""
     from orcaml_amd.backend import HipBackend
 
     rng = np.random.default_rng(M + 7 * K + N)
